@@ -109,13 +109,13 @@ def build_cpp_test() -> str | None:
 SANITIZE = ["-fsanitize=address,undefined", "-fno-sanitize-recover=all", "-fno-omit-frame-pointer"]
 
 
-def build_tile_test() -> str | None:
-    """The host tile-table builder's unit test (tests/cpp/test_tile_tables.cpp), built
+def build_tile_test(name: str = "test_tile_tables") -> str | None:
+    """A unit test of the host table builders (tests/cpp/<name>.cpp), built
     from the plain C++ builder sources with the sanitizers; needs no GPU."""
-    src = os.path.join(ROOT, "tests", "cpp", "test_tile_tables.cpp")
+    src = os.path.join(ROOT, "tests", "cpp", name + ".cpp")
     if not os.path.exists(src):
         return None
-    out = os.path.join(ROOT, "tests", "cpp", "test_tile_tables")
+    out = os.path.join(ROOT, "tests", "cpp", name)
     cxx = os.environ.get("CXX", "g++")
     _run([cxx, "-O1", "-g", "-std=c++20", "-Wall", "-Wextra", *SANITIZE, f"-I{INCLUDE}", f"-I{CSRC}",
           "-o", out + ".tmp", src, os.path.join(CSRC, "fp_tiles_host.cpp"), os.path.join(CSRC, "fp_error.cpp")])
@@ -125,7 +125,7 @@ def build_tile_test() -> str | None:
 
 def build_all() -> list[str]:
     built = [build_hip()]
-    for extra in (build_python(), build_cpp_test(), build_tile_test()):
+    for extra in (build_python(), build_cpp_test(), build_tile_test(), build_tile_test("test_column_tables")):
         if extra:
             built.append(extra)
     return built
@@ -141,5 +141,6 @@ if __name__ == "__main__":
         build_cpp_test()
     elif what == "tiletest":
         build_tile_test()
+        build_tile_test("test_column_tables")
     else:
         build_all()

@@ -1353,6 +1353,14 @@ fp_status fp_hip_op_expectation(fp_hip_ops const *ops, int dtype, void const *st
     if (st != FP_OK)
         return st;
     StreamGuard guard(static_cast<hipStream_t>(stream));
+    if (fprt::ev_columns_eligible(ops, dtype, n_states))
+    {
+        bool done = false;
+        st = fprt::run_op_expect_columns(ops, dtype, states, out, dim, n_states, accumulate,
+                                         static_cast<hipStream_t>(stream), nullptr, &done);
+        if (st != FP_OK || done)
+            return st;
+    }
     bool tiled = false;
     if ((st = fprt::choose_op_expect_tiled(ops, dtype, n_states, &tiled)) != FP_OK)
         return st;

@@ -76,6 +76,13 @@ extern "C" fp_status fp_hip_op_expectation_noalloc(fp_hip_ops const *ops, int dt
     }
     Workspace const ws{base, kScratchBytes};
     hipStream_t const s = static_cast<hipStream_t>(stream);
+    if (ev_columns_eligible(ops, dtype, n_states))
+    {
+        bool done = false;
+        st = run_op_expect_columns(ops, dtype, states, out, dim, n_states, accumulate, s, &ws, &done);
+        if (st != FP_OK || done)
+            return st;
+    }
     bool tiled = false;
     if ((st = choose_op_expect_tiled(ops, dtype, n_states, &tiled)) != FP_OK)
         return st;

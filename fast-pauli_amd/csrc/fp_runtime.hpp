@@ -185,6 +185,12 @@ fp_status run_op_expect_tiled(fp_hip_ops const *ops, int dtype, void const *stat
 fp_status run_op_expect(fp_hip_ops const *ops, int dtype, void const *states, void *out, size_t dim, size_t n_states,
                         size_t s_begin, size_t count, double const *scale_table, double post_re, double post_im,
                         int accumulate, hipStream_t st, Workspace const *ws = nullptr);
+// PauliOp expectation on state columns (fp_columns.hpp).  *done = false, with nothing
+// enqueued, when it cannot run here (no room for the transposed slab in the workspace or on
+// the device, or the stream is being captured): the caller takes another kernel.
+bool ev_columns_eligible(fp_hip_ops const *ops, int dtype, size_t n_states);
+fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *states, void *out, size_t dim,
+                                size_t n_states, int accumulate, hipStream_t st, Workspace const *ws, bool *done);
 // Shape checks shared by the entry points.
 fp_status check_shape(fp_hip_ops const *ops, int dtype, void const *a, void const *b, size_t dim, size_t n_states);
 // Sets up the allocation-free entry point's static buffer on the current device

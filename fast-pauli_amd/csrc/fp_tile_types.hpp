@@ -166,3 +166,73 @@ struct EvStr
 };
 
 } // namespace fpl
+
+// PauliOp expectation on state columns (the column kernel).  A column's rows are cut
+// into tiles of 2^w consecutive rows; within a tile a row index is
+//   [wave bits | 3 slot bits | 6 lane bits | sub bit (complex64 only)],
+// the slots being the 8 16-byte pieces (one complex128 or two complex64 rows) a thread owns.
+// Strings are filed by class u = x >> w: a class pairs leader tile p with tile p ^ u.
+namespace fpc
+{
+
+constexpr uint32_t kSlotBits = 3;
+constexpr uint32_t kLaneBits = 6;
+constexpr uint32_t kThreads = 512;
+constexpr uint32_t kWaveBits = 3;
+constexpr uint32_t kTileBytes = kThreads * 8u * 16u;
+
+FP_HD constexpr uint32_t sub_bits(bool c64)
+{
+    return c64 ? 1u : 0u;
+}
+// row bits below the wave bits
+FP_HD constexpr uint32_t low_bits(bool c64)
+{
+    return kSlotBits + kLaneBits + sub_bits(c64);
+}
+FP_HD constexpr uint32_t tile_bits(bool c64)
+{
+    return kWaveBits + low_bits(c64);
+}
+
+// One block's work on a column: leader tile p, entries [entry_first, entry_first + entry_count).
+struct ColItem
+{
+    uint32_t p;
+    uint32_t entry_first;
+    uint32_t entry_count;
+    uint32_t pad;
+};
+
+// Strings [first, first + count) of class u: the partner tile is p ^ u.
+struct ColEntry
+{
+    uint32_t u;
+    uint32_t first;
+    uint32_t count;
+    uint32_t pad;
+};
+
+// ColStr::code: bits 0-2 the slot bits of x, bit 3 its sub bit, bit 4 Im w, and one of
+//   bit 5: x = 0 (every row, |psi|^2),
+//   bit 6: partner in the same tile, pairs led by the slots whose bit (the highest slot
+//          bit of x) is clear;
+// bits 8-10 the slot bits of z, bit 11 its sub bit.  A same-tile string whose slot bits are
+// all clear visits each pair from both sides (its scale is halved).
+constexpr uint32_t kColSub = 8, kColImag = 16, kColSelf = 32, kColHalf = 64, kColCase = 127;
+constexpr uint32_t kColZShift = 8;
+// bits 16 up: how many strings of the class, from this one on, share its case
+constexpr uint32_t kColRunShift = 16, kColRunMax = 0xffff;
+
+struct ColStr
+{
+    uint32_t px;   // byte offset of x's lane and wave bits within the tile (XOR)
+    uint32_t zl;   // z's lane bits
+    uint32_t zg;   // z's bits above the slot bits
+    uint32_t code;
+    double sre; // scale c_s * kappa_s (times 1/2 where pairs are visited twice)
+    double sim;
+};
+
+} // namespace fpc
+

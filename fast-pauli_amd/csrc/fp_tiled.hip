@@ -78,7 +78,8 @@ fp_status tile_tables(fp_hip_ops const *ops, int kind, uint32_t k, uint32_t dh, 
     StringTable const st{ops->n_qubits, ops->n_strings, ops->x.data(), ops->z.data(), ops->ny.data(),
                          ops->coeffs.data(), c128, c64};
     TileImage img;
-    fp_status const bs = build_tile_image(st, kind, k, dh, wht_min, img);
+    fp_status const bs = kind == kTilesEvColumns ? build_column_image(st, dh != 0, k, img)
+                                                 : build_tile_image(st, kind, k, dh, wht_min, img);
     if (bs != FP_OK)
         return bs;
 

@@ -554,4 +554,144 @@ fp_status build_tile_image(StringTable const &table, int kind, uint32_t k, uint3
     return FP_OK;
 }
 
+namespace
+{
+
+struct ColClass
+{
+    uint64_t u;
+    uint32_t lead; // leader tiles have this bit of p clear (classes u != 0)
+    std::vector<fpc::ColStr> strs;
+};
+
+// One record and its class.  The pair sum is the same whichever row of a pair leads it.
+fpc::ColStr column_record(StringTable const &st, bool c64, size_t s, uint64_t &u)
+{
+    uint32_t const sb = fpc::sub_bits(c64), lb = fpc::kLaneBits, low = fpc::low_bits(c64);
+    uint64_t const x = st.x[s], z = st.z[s];
+    uint32_t const lanes = (1u << lb) - 1u;
+    u = x >> fpc::tile_bits(c64);
+    uint32_t const xs = uint32_t(x >> (sb + lb)) & 7u, zs = uint32_t(z >> (sb + lb)) & 7u;
+    uint32_t const x_wave = uint32_t(x >> low) & ((1u << fpc::kWaveBits) - 1u);
+    fpc::ColStr r{};
+    r.px = (x_wave << (fpc::kSlotBits + lb + 4u)) | ((uint32_t(x >> sb) & lanes) << 4u);
+    r.zl = uint32_t(z >> sb) & lanes;
+    r.zg = uint32_t(z >> low);
+    r.code = xs | (sb && (x & 1u) ? fpc::kColSub : 0u) | ((st.ny[s] & 1u) ? fpc::kColImag : 0u) |
+             (zs << fpc::kColZShift) | (sb && (z & 1u) ? 8u << fpc::kColZShift : 0u);
+    double kap = kappa_of(x, st.ny[s]);
+    if (x == 0)
+        r.code |= fpc::kColSelf;
+    else if (u == 0)
+    {
+        if (xs)
+            r.code |= fpc::kColHalf;
+        else
+            kap *= 0.5; // exact
+    }
+    r.sre = st.coeffs[2 * s] * kap;
+    r.sim = st.coeffs[2 * s + 1] * kap;
+    return r;
+}
+
+double record_cost(fpc::ColStr const &r)
+{
+    return (r.code & fpc::kColHalf) ? 0.6 : 1.0;
+}
+
+} // namespace
+
+fp_status build_column_image(StringTable const &st, bool c64, uint32_t per_item, TileImage &out)
+{
+    uint32_t const w = fpc::tile_bits(c64);
+    size_t const n = st.n_qubits;
+    if (n < fpc::low_bits(c64) || n > w + 12u)
+        return fail(FP_ERR_RUNTIME, "the column tables take %u to %u qubits (got %zu)", fpc::low_bits(c64), w + 12, n);
+    std::vector<ColClass> classes;
+    {
+        std::vector<std::pair<uint64_t, fpc::ColStr>> rec(st.n_strings);
+        for (size_t s = 0; s < st.n_strings; ++s)
+            rec[s].second = column_record(st, c64, s, rec[s].first);
+        // by class; within a class by case (one body after the other), then by partner rows
+        std::stable_sort(rec.begin(), rec.end(), [](auto const &a, auto const &b) {
+            uint32_t const ca = a.second.code & fpc::kColCase, cb = b.second.code & fpc::kColCase;
+            return a.first != b.first ? a.first < b.first : (ca != cb ? ca < cb : a.second.px < b.second.px);
+        });
+        for (auto const &r : rec)
+        {
+            if (classes.empty() || classes.back().u != r.first)
+            {
+                // any set bit of u may choose the leaders; spread the choice over the classes
+                ColClass c{r.first, 0, {}};
+                if (c.u)
+                {
+                    uint32_t skip = uint32_t(classes.size()) % uint32_t(__builtin_popcountll(c.u));
+                    uint64_t v = c.u;
+                    while (skip--)
+                        v &= v - 1;
+                    c.lead = uint32_t(__builtin_ctzll(v));
+                }
+                classes.push_back(std::move(c));
+            }
+            classes.back().strs.push_back(r.second);
+        }
+    }
+    std::vector<fpc::ColStr> strs;
+    std::vector<fpc::ColEntry> entries;
+    std::vector<fpc::ColItem> items;
+    std::vector<uint32_t> first(classes.size());
+    for (size_t c = 0; c < classes.size(); ++c)
+    {
+        first[c] = uint32_t(strs.size());
+        auto &cs = classes[c].strs;
+        uint32_t run = 0; // stretches of one case, counted from the back
+        for (size_t i = cs.size(); i-- > 0;)
+        {
+            bool const same = i + 1 < cs.size() && ((cs[i].code ^ cs[i + 1].code) & fpc::kColCase) == 0;
+            run = same ? std::min(run + 1, fpc::kColRunMax) : 1u;
+            cs[i].code |= run << fpc::kColRunShift;
+        }
+        strs.insert(strs.end(), cs.begin(), cs.end());
+    }
+    strs.push_back(fpc::ColStr{}); // read ahead of the last string
+    uint64_t const tiles = n > w ? uint64_t(1) << (n - w) : 1u;
+    double const limit = std::max<uint32_t>(per_item, 1);
+    for (uint64_t p = 0; p < tiles; ++p)
+    {
+        double cost = limit; // the first entry opens an item
+        for (size_t c = 0; c < classes.size(); ++c)
+        {
+            ColClass const &cl = classes[c];
+            if (cl.u && ((p >> cl.lead) & 1u))
+                continue;
+            for (size_t i = 0; i < cl.strs.size();)
+            {
+                if (cost >= limit)
+                {
+                    items.push_back(fpc::ColItem{uint32_t(p), uint32_t(entries.size()), 0, 0});
+                    cost = 0.0;
+                }
+                size_t j = i;
+                while (j < cl.strs.size() && cost < limit)
+                    cost += record_cost(cl.strs[j++]);
+                entries.push_back(fpc::ColEntry{uint32_t(cl.u), uint32_t(first[c] + i), uint32_t(j - i), 0});
+                ++items.back().entry_count;
+                i = j;
+            }
+        }
+    }
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    out.n_groups = uint32_t(items.size());
+    out.max_chunks = 0;
+    out.o_btab = up(items.size() * sizeof(fpc::ColItem));
+    out.o_chunks = out.o_btab;
+    out.o_strs = out.o_chunks + up(entries.size() * sizeof(fpc::ColEntry));
+    out.o_sh = out.o_strs + up(strs.size() * sizeof(fpc::ColStr));
+    out.h.assign(out.o_sh, 0);
+    std::memcpy(out.h.data(), items.data(), items.size() * sizeof(fpc::ColItem));
+    std::memcpy(out.h.data() + out.o_chunks, entries.data(), entries.size() * sizeof(fpc::ColEntry));
+    std::memcpy(out.h.data() + out.o_strs, strs.data(), strs.size() * sizeof(fpc::ColStr));
+    return FP_OK;
+}
+
 } // namespace fprt

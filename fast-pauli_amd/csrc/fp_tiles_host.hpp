@@ -31,6 +31,8 @@ enum
     kTilesOpApply = 2,  // fpa::ApplyStr records, groups of consecutive strings (PauliOp apply)
     kTilesSummedApply = 3, // the same for SummedPauliOp::apply: StringTable::cf128 / cf64 hold the
                            // folded row sums of the coefficient matrix
+    kTilesEvColumns = 5, // fpc:: records (PauliOp expectation on state columns): groups hold the
+                         // items, chunks the entries
     kTilesWeightedApply = 4 // the same for SummedPauliOp::apply_weighted: StringTable::cf128 / cf64
                             // hold (-i)^{nY} (the per-state weights are applied in the kernel)
 };
@@ -74,5 +76,11 @@ struct TileImage
 // equal half of w become transform classes (listed first in each group).
 fp_status build_tile_image(StringTable const &st, int kind, uint32_t k, uint32_t dh, uint32_t wht_min,
                            TileImage &out);
+
+// Items, entries and string records of the expectation column kernel (kTilesEvColumns):
+// fpc::ColItem at offset 0, fpc::ColEntry at o_chunks, fpc::ColStr at o_strs.  Strings are
+// filed by x >> tile_bits; each leader tile's entries are cut into items of about `per_item`
+// string evaluations of a whole tile (n_groups items).
+fp_status build_column_image(StringTable const &st, bool c64, uint32_t per_item, TileImage &out);
 
 } // namespace fprt

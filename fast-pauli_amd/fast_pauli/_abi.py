@@ -86,6 +86,7 @@ _SIGS = {
     "fp_hip_op_apply": [_vp, _i, _vp, _vp, _sz, _sz, _i, _vp],
     "fp_hip_op_expectation": [_vp, _i, _vp, _vp, _sz, _sz, _i, _vp],
     "fp_hip_op_expectation_plan": [_vp, _i, _sz, _sz, _vp],
+    "fp_hip_op_expectation_columns": [_vp, _i, _sz, _sz, ctypes.POINTER(_i)],
     "fp_hip_op_apply_plan": [_vp, _i, _sz, _sz, _i, _vp],
     "fp_hip_summed_apply_plan": [_vp, _i, _sz, _sz, _i, _vp],
     "fp_hip_summed_apply_weighted_plan": [_vp, _i, _sz, _sz, _i, _vp],
@@ -116,8 +117,15 @@ class EvPlan(ctypes.Structure):
         return {f: int(getattr(self, f)) for f, _ in self._fields_}
 
 
+def op_expectation_columns(ops, dtype: int, dim: int, n_states: int) -> bool:
+    """Whether fp_hip_op_expectation evaluates these shapes on state columns."""
+    c = _i(0)
+    call("fp_hip_op_expectation_columns", ops.handle, dtype, dim, n_states, ctypes.byref(c))
+    return bool(c.value)
+
+
 def op_expectation_plan(ops, dtype: int, dim: int, n_states: int) -> dict:
-    """Which kernel fp_hip_op_expectation runs for these shapes, and its HBM bytes."""
+    """The row-major kernel of fp_hip_op_expectation for these shapes, and its HBM bytes."""
     p = EvPlan()
     call("fp_hip_op_expectation_plan", ops.handle, dtype, dim, n_states, ctypes.byref(p))
     return p.as_dict()

@@ -165,14 +165,24 @@ fp_status fp_hip_op_apply(fp_hip_ops const *ops, int dtype, void const *states, 
 fp_status fp_hip_op_expectation(fp_hip_ops const *ops, int dtype, void const *states, void *out, size_t dim,
                                 size_t n_states, int accumulate, void *stream);
 
+/* Whether fp_hip_op_expectation (and _noalloc) evaluates these shapes on state columns: each
+ * state made one contiguous column (a transposed copy in the stream's scratch, at most 128 MiB
+ * at a time; a single aligned state as it is), tiles of it held in registers and LDS.  No
+ * counterpart in the reference.  Where the copy has no room (device memory, or the static
+ * workspace), and in fp_hip_op_expectation on a stream that is being captured, the call runs
+ * the kernel of fp_hip_op_expectation_plan instead. */
+fp_status fp_hip_op_expectation_columns(fp_hip_ops const *ops, int dtype, size_t dim, size_t n_states,
+                                        int *columns);
+
 /* Size of the static device workspace of fp_hip_op_expectation_noalloc (per GPU). */
 #define FP_NOALLOC_SCRATCH_BYTES ((size_t)32 << 20)
 
 /* fp_hip_op_expectation without any device allocation.  No counterpart in the reference: it is
  * for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  Same kernels, same results as fp_hip_op_expectation (identical bits
- * whenever the partials fit beside the tables without fewer blocks; otherwise a regrouped FP64
- * sum); the reduction partials and the string-group tables live in one static
+ * whenever the partials, and on state columns the transposed states, fit beside the tables
+ * without fewer blocks or another kernel; otherwise a regrouped FP64 sum); the reduction
+ * partials, the transposed states and the string-group tables live in one static
  * FP_NOALLOC_SCRATCH_BYTES device array per GPU instead of library-allocated memory.  Shapes
  * whose tables and partials (tiled: groups x n_states x 16 B at least; streaming:
  * n_states x 16 B at least) exceed it fail with FP_ERR_INVALID_ARGUMENT before any kernel runs.
@@ -183,8 +193,9 @@ fp_status fp_hip_op_expectation(fp_hip_ops const *ops, int dtype, void const *st
 fp_status fp_hip_op_expectation_noalloc(fp_hip_ops const *ops, int dtype, void const *states, void *out,
                                         size_t dim, size_t n_states, int accumulate, void *stream);
 
-/* How fp_hip_op_expectation evaluates these shapes.  No counterpart in the reference:
- * diagnostics and roofline accounting for callers that measure the kernel.
+/* How fp_hip_op_expectation evaluates these shapes on the row-major batch itself, which it does
+ * unless fp_hip_op_expectation_columns says that it takes state columns.  No counterpart in the
+ * reference: diagnostics and roofline accounting for callers that measure the kernel.
  *   kernel 0 (FP_EV_STREAM): every string reads the whole state once.
  *   kernel 1 (FP_EV_TILED):  strings are grouped so that the x masks of a group span a subspace
  *     of dimension tile_rows_log2 (with its low bits); each coset of it is a tile of
