@@ -538,6 +538,7 @@ def bench_op_apply_n24(args) -> dict:
                       3)
         gbs = plan["hbm_bytes"] / (ms / 1e3) / 1e9
         res[name] = {"ms": ms, "strings_x_states_per_s": N * S / (ms / 1e3), "plan": plan,
+                     "columns": _abi.op_apply_columns(ops, dt, 1 << n, S),
                      "achieved_gbs": gbs, "frac_hbm": gbs / HBM_PEAK_GBS,
                      "streaming_model_bytes": (N + 1) * (1 << n) * S * esz}
         if dt == _abi.FP_C128:
@@ -612,8 +613,10 @@ def bench_summed_n14(args) -> dict:
 def bench_summed_apply_n14(args, failures) -> dict:
     """SummedPauliOp::apply and apply_weighted on the n=14 operator set (2000 strings of
     weight <= 3, 200 operators) and 1000 states, complex128: every output element sums its
-    2000 strings' terms in order, through the coset-tiled kernel (string groups sharing LDS
-    tiles) where its plan pays, else the streaming kernels (one partner read per string)."""
+    2000 strings' terms in order, on state columns (one launch for all strings) where the rule
+    takes them, else through the coset-tiled kernel (string groups sharing LDS tiles) where its
+    plan pays, else the streaming kernels (one partner read per string).  The plan's bytes are
+    those of the row-major kernels and give no rate for a run on columns."""
     from fast_pauli import _abi, synthetic as syn
 
     n, N, K, S = 14, 2000, 200, 1000
@@ -633,17 +636,25 @@ def bench_summed_apply_n14(args, failures) -> dict:
     model = (N + 1) * state_bytes  # streaming: one partner read per string, one output write
     plan = _abi.summed_apply_plan(ops, _abi.FP_C128, dim, S)
     wplan = _abi.summed_apply_weighted_plan(ops, _abi.FP_C128, dim, S)
+    col, wcol = (_abi.op_apply_columns(ops, _abi.FP_C128, dim, S, w) for w in (False, True))
+
+    def kernel(on_columns, p):
+        return "columns" if on_columns else "coset-tiled" if p["kernel"] == _abi.FP_EV_TILED else "streaming"
+
+    def gbs(on_columns, p, ms):
+        return None if on_columns else p["hbm_bytes"] / (ms / 1e3) / 1e9
+
+    rate = gbs(col, plan, ms_apply)
     res = {"config": "n=14, 2000 strings of weight <= 3, h (2000 x 200) ~ N(0,1) real, x (200 x 1000) ~ N(0,1), "
                      "1000 normalised states, complex128",
            "apply_ms": ms_apply, "apply_weighted_ms": ms_w,
-           "apply_kernel": "coset-tiled" if plan["kernel"] == _abi.FP_EV_TILED else "streaming",
+           "apply_kernel": kernel(col, plan),
            "apply_groups": plan["n_groups"], "apply_plan_bytes": plan["hbm_bytes"],
-           "apply_plan_gbs": plan["hbm_bytes"] / (ms_apply / 1e3) / 1e9,
-           "apply_plan_frac_hbm": plan["hbm_bytes"] / (ms_apply / 1e3) / 1e9 / HBM_PEAK_GBS,
+           "apply_plan_gbs": rate, "apply_plan_frac_hbm": rate / HBM_PEAK_GBS if rate else None,
            "streaming_model_bytes": model, "streaming_bytes_rule": "(strings + 1) x 2^n x S x 16 B",
-           "apply_weighted_kernel": "coset-tiled" if wplan["kernel"] == _abi.FP_EV_TILED else "streaming",
+           "apply_weighted_kernel": kernel(wcol, wplan),
            "apply_weighted_plan_bytes": wplan["hbm_bytes"],
-           "apply_weighted_plan_gbs": wplan["hbm_bytes"] / (ms_w / 1e3) / 1e9,
+           "apply_weighted_plan_gbs": gbs(wcol, wplan, ms_w),
            "strings_x_states_per_s": N * S / (ms_apply / 1e3)}
     if not args.no_cpu:
         from oracle import oracle as O

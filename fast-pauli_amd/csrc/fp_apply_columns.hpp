@@ -1,0 +1,303 @@
+// fp_apply_columns.hpp — PauliOp::apply (and SummedPauliOp::apply / apply_weighted) on state
+// columns, bit-exact with the sequential string order.
+//
+// A column is a contiguous array of 2^n rows of one state (complex64: of two neighbouring
+// states, 16 bytes a row): a transposed copy of the batch, or the batch itself when its row
+// length is a power of two (a row-major batch of 2^k states is one column of 2^(n + k) rows on
+// which every mask is shifted by k).  Each thread owns E rows, 64 apart, keeps their sums in
+// registers and adds the strings in order, so every element sees the sequential loop's
+// operations (cmul_exact, one rounding per sum) in its order: one launch for all strings, the
+// column read once per string from L2 or LDS and written once.
+//
+// The partner of row (g, i, lane) (wave, slot, lane parts) is (g ^ x_g, i ^ x_i, lane ^ x_l):
+// a per-lane offset (one XOR per string), a scalar offset per slot.  The sign is a per-lane bit,
+// a wave-uniform bit and one flip per slot, applied as the factor of the final multiply-add.
+//
+// Bound: about 10 vector instructions per (string, 64 rows), 8 of them the unfused product and
+// sums, against 16 clocks of L1 for a gathered KiB (64 bytes a clock; 4 clocks from LDS).  Two
+// shapes are built: one row a thread, partner rows gathered from L2 four strings ahead; and 2^13
+// rows a block in LDS (fp_columns.hip says which runs where).  Measured, row-major kernels /
+// columns, us: n = 10, 128 complex128 states, 64 strings 18.6 / 10.9; n = 18, one complex128
+// state, 1000 strings 287 / 144; n = 20, 19 complex64 states, 512 strings 10990 / 5780 (8 MiB a
+// column: past an XCD's L2); n = 14, 1000 complex128 states, 2000 strings, a weight per string
+// and state 29130 / 11520.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "fp_columns.hpp"
+#include "fp_kernels.hpp"
+
+namespace fpc
+{
+
+// A uniform pointer held in scalar registers (the compiler cannot always tell).
+template <class P> __device__ __forceinline__ P const *uniform(P const *p)
+{
+    uint64_t const v = reinterpret_cast<uint64_t>(p);
+    uint32_t const lo = __builtin_amdgcn_readfirstlane(uint32_t(v));
+    uint32_t const hi = __builtin_amdgcn_readfirstlane(uint32_t(v >> 32));
+    return reinterpret_cast<P const *>((uint64_t(hi) << 32) | lo);
+}
+
+// Buffer over one column of `rows` pieces; reads past its end return zero.
+template <class V> __device__ __forceinline__ __amdgpu_buffer_rsrc_t column_rsrc(V const *col, uint64_t rows)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<V *>(uniform(col)), short(0),
+                                             int(uint32_t(rows * sizeof(V))), 0x00027000);
+}
+
+template <class V> __device__ __forceinline__ V buffer_load(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff)
+{
+    if constexpr (sizeof(V) == 16)
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, int(voff), int(soff), 0));
+    else
+        return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rsrc, int(voff), int(soff), 0));
+}
+
+// +-1 with the sign in bit 31 of `bits` (other bits clear)
+template <class T> __device__ __forceinline__ T unit_sign(uint32_t bits)
+{
+    if constexpr (sizeof(T) == 8)
+        return __hiloint2double(int(bits | 0x3ff00000u), 0);
+    else
+        return __uint_as_float(bits | 0x3f800000u);
+}
+// v with its sign flipped by bit 31 of `bits`
+template <class T> __device__ __forceinline__ T flip(T v, uint32_t bits)
+{
+    if constexpr (sizeof(T) == 8)
+        return __hiloint2double(__double2hiint(v) ^ int(bits), __double2loint(v));
+    else
+        return __uint_as_float(__float_as_uint(v) ^ bits);
+}
+
+constexpr uint32_t log2c(uint32_t v)
+{
+    return v <= 1 ? 0 : 1 + log2c(v / 2);
+}
+
+// Records read past the last string (the tables are padded by as many).
+constexpr uint32_t kXzPad = 64;
+
+// cols, out: n_cols columns of 2^n rows; NS states a row.  A block of TH threads owns a tile of
+// TH * E rows of a column, or the columns that fill it (n_groups * tiles blocks).
+// LDS: the tile's rows are kept in LDS, and strings whose partner rows lie in it read them there.
+// PIPE: the next strings' partner rows are in flight while U strings are added.
+// cf: complex coefficients with (-i)^{nY} folded in; WTD: those of state t at cf + 2 * cf_stride * t.
+// shift: masks are shifted by this many bits (one column made of a whole batch).
+template <class T, int NS, int E, int U, int TH, bool LDS, bool PIPE, bool WTD>
+__global__ __launch_bounds__(TH) void k_apply_columns(typename fpk::VecOf<T, NS>::type const *__restrict__ cols,
+                                                      typename fpk::VecOf<T, NS>::type *__restrict__ out, uint32_t n,
+                                                      uint32_t n_cols, uint32_t n_groups, uint32_t tiles,
+                                                      XZ const *__restrict__ xz, T const *__restrict__ cf,
+                                                      uint64_t cf_stride, uint32_t n_states, uint32_t n_strings, uint32_t shift,
+                                                      int accumulate)
+{
+    typedef typename fpk::VecOf<T, NS>::type V; // one row of NS states
+    constexpr uint32_t kLe = log2c(E), kLv = log2c(sizeof(V));
+    constexpr uint32_t kLow = 6u + kLe;                // row bits inside a wave
+    constexpr uint32_t kTile = kLow + log2c(TH / 64u); // log2 rows of a tile
+    constexpr uint32_t kSlot = 64u * sizeof(V);        // bytes from one slot to the next
+    extern __shared__ __align__(16) unsigned char smem[];
+    uint32_t const lane = threadIdx.x & 63u;
+    uint32_t const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    BlockOf const bo = block_of(blockIdx.x, tiles, n_groups);
+    uint32_t const grp = bo.group, p = bo.index;
+    uint32_t const per = n < kTile ? 1u << (kTile - n) : 1u; // columns in a tile
+    uint64_t const rows = uint64_t(1) << n;
+    uint32_t const t = grp * per + (n < kTile ? (wave << kLow) >> n : 0u);
+    if (!LDS && t >= n_cols)
+        return;
+    bool const live = t < n_cols; // a ragged last group has dead waves
+    uint32_t const tc = live ? t : n_cols - 1u;
+    V const *col = cols + uint64_t(tc) * rows;
+    // this thread's rows of the column: row0 + 64 i
+    uint32_t const g = n < kTile ? wave & ((1u << (n - kLow)) - 1u) : (p << (kTile - kLow)) | wave; // row >> kLow
+    uint32_t const row0 = (g << kLow) | lane;
+    V *oc = out + uint64_t(tc) * rows + row0;
+    uint32_t const a0 = ((wave << kLow) | lane) << kLv; // LDS address of slot 0
+    if constexpr (LDS)
+    {
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+            *reinterpret_cast<V *>(smem + a0 + uint32_t(i) * kSlot) = col[row0 + uint32_t(i) * 64u];
+    }
+    V acc[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+        acc[i] = accumulate && live ? oc[i * 64] : V(0);
+    if constexpr (LDS)
+        __syncthreads();
+    // WTD: the coefficients of this column's states (the last state again past the end)
+    T const *c[WTD ? NS : 1];
+#pragma unroll
+    for (int w = 0; w < (WTD ? NS : 1); ++w)
+        c[w] = cf + 2 * cf_stride * (WTD ? (tc * NS + w < n_states ? tc * NS + w : n_states - 1u) : 0u);
+    __amdgpu_buffer_rsrc_t const rsrc = column_rsrc(col, rows);
+    uint32_t const lv = lane << kLv, gv = g << (kLow + kLv);
+    // Three stages: the records of batch k + 2 (scalar loads), the partner rows of batch
+    // k + 1, the terms of batch k.  Records past the end are read (the tables are padded)
+    // and their partner rows too (inside the column, or zero), but add nothing.
+    struct Rec
+    {
+        XZ q;
+        T cr[WTD ? NS : 1], ci[WTD ? NS : 1];
+    };
+    Rec rec[3][U];
+    V R[PIPE ? 2 : 1][U][E];
+    XZ const *qp = xz;
+    auto fetch = [&](int k, Rec(&r)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            r[u].q = XZ{qp[k * U + u].x << shift, qp[k * U + u].z << shift};
+#pragma unroll
+            for (int w = 0; w < (WTD ? NS : 1); ++w)
+            {
+                r[u].cr[w] = c[w][2 * (k * U + u)];
+                r[u].ci[w] = c[w][2 * (k * U + u) + 1];
+            }
+        }
+    };
+    auto load = [&](Rec const(&r)[U], V(&v)[U][E]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+        {
+            uint32_t const x = r[u].q.x;
+            if (LDS && (x >> kTile) == 0)
+            {
+                uint32_t const a = a0 ^ (x << kLv);
+#pragma unroll
+                for (int i = 0; i < E; ++i)
+                    v[u][i] =
+                        *reinterpret_cast<__attribute__((address_space(3))) V const *>(a ^ (uint32_t(i) * kSlot));
+            }
+            else
+            {
+                uint32_t const vo = lv ^ ((x & 63u) << kLv), so = gv ^ ((x >> 6) << (6u + kLv));
+#pragma unroll
+                for (int i = 0; i < E; ++i)
+                    v[u][i] = buffer_load<V>(rsrc, vo, so ^ (uint32_t(i) * kSlot));
+            }
+        }
+    };
+    auto eval = [&](uint32_t s0, Rec const(&r)[U], V(&v)[U][E]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s0 + uint32_t(u) < n_strings)
+            {
+                uint32_t const z = r[u].q.z;
+                // sign of the row: per-lane bits, wave-uniform bits, then one flip per slot
+                uint32_t const neg = uint32_t(__popc(lane & z)) + uint32_t(__popc(g & (z >> kLow)));
+                uint32_t zb[kLe + 1];
+#pragma unroll
+                for (uint32_t b = 0; b < kLe; ++b)
+                    zb[b] = (z << (25u - b)) & 0x80000000u;
+                T sg = unit_sign<T>(neg << 31);
+                // slots in Gray-code order: one sign flip from each to the next
+#pragma unroll
+                for (int j = 0; j < E; ++j)
+                {
+                    int const i = j ^ (j >> 1);
+                    if (j)
+                        sg = flip<T>(sg, zb[__builtin_ctz(uint32_t(j))]);
+#pragma unroll
+                    for (int h = 0; h < NS; ++h)
+                    {
+                        // the signed term: products and their sum rounded as cmul_exact does, then
+                        // one rounding in the sum, which a multiply-add by +-1 gives exactly
+                        int const w = WTD ? h : 0;
+                        T tr, ti;
+                        fpk::cmul_exact<T>(r[u].cr[w], r[u].ci[w], v[u][i][2 * h], v[u][i][2 * h + 1], tr, ti);
+                        acc[i][2 * h] = fma(sg, tr, acc[i][2 * h]);
+                        acc[i][2 * h + 1] = fma(sg, ti, acc[i][2 * h + 1]);
+                    }
+                }
+            }
+    };
+    fetch(0, rec[0]);
+    fetch(1, rec[1]);
+    if constexpr (PIPE)
+        load(rec[0], R[0]);
+    for (uint32_t s0 = 0; s0 < n_strings; s0 += 6 * U)
+    {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) // a multiple of both buffer counts
+        {
+            uint32_t const sk = s0 + uint32_t(k) * U;
+            if (sk >= n_strings)
+                break;
+            fetch(k + 2, rec[(k + 2) % 3]);
+            if constexpr (PIPE)
+            {
+                if (sk + U < n_strings)
+                    load(rec[(k + 1) % 3], R[(k + 1) % 2]);
+            }
+            else
+                load(rec[k % 3], R[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            eval(sk, rec[k % 3], R[PIPE ? k % 2 : 0]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        qp += 6 * U;
+#pragma unroll
+        for (int w = 0; w < (WTD ? NS : 1); ++w)
+            c[w] += 12 * U;
+    }
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+        if (live)
+            __builtin_nontemporal_store(acc[i], oc + i * 64);
+}
+
+// w(s, t) = sum_k h(s, k) x(k, t), k in order, product then add (no contraction: the reference's
+// sequential loop, fast_pauli/cpp/include/__summed_pauli_op.hpp:378-503), times (-i)^{nY_s} (an
+// exact swap and negation), one row of n_strings per state.  A thread takes one state and R
+// strings, whose h are scalar loads: x is read once for R sums (one string a thread read it N
+// times: 406 us at 2000 strings, 200 operators, 1000 states).
+template <class T, int R>
+__global__ __launch_bounds__(256) void k_weights(T const *__restrict__ h, T const *__restrict__ x,
+                                                 uint32_t const *__restrict__ nys, T *__restrict__ w,
+                                                 uint64_t n_strings, uint64_t n_ops, uint64_t n_states)
+{
+#pragma clang fp contract(off)
+    uint64_t const t = uint64_t(blockIdx.x) * 256 + threadIdx.x;
+    uint64_t const s0 = uint64_t(blockIdx.y) * R;
+    if (t >= n_states)
+        return;
+    T wr[R], wi[R];
+    T const *hp[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+    {
+        wr[r] = wi[r] = T(0);
+        hp[r] = h + 2 * n_ops * (s0 + r < n_strings ? s0 + r : n_strings - 1);
+    }
+    for (uint64_t k = 0; k < n_ops; ++k)
+    {
+        T const d = x[k * n_states + t];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+        {
+            T const pr = hp[r][2 * k] * d;
+            T const pi = hp[r][2 * k + 1] * d;
+            wr[r] = wr[r] + pr;
+            wi[r] = wi[r] + pi;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (s0 + r < n_strings)
+        {
+            uint32_t const ny = nys[s0 + r] & 3u;
+            T const a = wr[r], b = wi[r];
+            w[2 * (t * n_strings + s0 + r)] = ny == 0 ? a : ny == 1 ? b : ny == 2 ? -a : -b;
+            w[2 * (t * n_strings + s0 + r) + 1] = ny == 0 ? b : ny == 1 ? -a : ny == 2 ? -b : a;
+        }
+}
+
+} // namespace fpc

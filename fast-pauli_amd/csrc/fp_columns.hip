@@ -5,9 +5,11 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 
 #include "fast_pauli_hip.h"
+#include "fp_apply_columns.hpp"
 #include "fp_columns.hpp"
 #include "fp_runtime.hpp"
 
@@ -58,6 +60,14 @@ ColGeom col_geom(fp_hip_ops const *ops, int dtype, size_t n_states, size_t slab_
         cols = std::max<size_t>(cols / (8 * g.per_group) * (8 * g.per_group), std::min<size_t>(cols, g.per_group));
     g.slab = uint32_t(std::min<size_t>(cols, 0x7fffffffu));
     return g;
+}
+
+template <class T, int NS, bool IN>
+void launch_columns(typename fpk::VecOf<T, 1>::type *batch, typename fpk::VecOf<T, NS>::type *cols, uint64_t rows,
+                    uint64_t ld, uint64_t c0, uint32_t n_cols, hipStream_t st)
+{
+    dim3 const grid(uint32_t((rows + 31) / 32), (n_cols + 31) / 32);
+    hipLaunchKernelGGL((fpc::k_columns<T, NS, IN>), grid, dim3(256), 0, st, batch, cols, rows, ld, c0, n_cols);
 }
 
 } // namespace
@@ -124,10 +134,7 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
     if (s != FP_OK)
         return s;
     uint32_t const n_items = tt->n_groups;
-    // from 4 column groups per XCD: their items stay on one XCD, whose L2 then serves the tiles
-    // (n = 16 S = 40 N = 300 complex64: 82 us against 86)
-    bool const xcd = n_groups_max >= 32;
-    if (uint64_t(n_items) * (n_groups_max + 8) > 0x7fffffffu)
+    if (uint64_t(n_items) * n_groups_max > 0x7fffffffu)
         return FP_OK;
     size_t const slab_bytes = in_place ? 0 : round256(size_t(g.slab) * g.col_bytes);
     size_t const part_bytes = round256(size_t(n_items) * g.slab * sizeof(fpk::Dbl2));
@@ -180,16 +187,15 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
             P const *cols = static_cast<P const *>(states);
             if (!in_place)
             {
-                dim3 const tg(uint32_t((dim + 31) / 32), (nc + 31) / 32);
-                hipLaunchKernelGGL(fpc::k_columns_in<V>, tg, dim3(256), 0, st, static_cast<V const *>(states),
-                                   reinterpret_cast<V *>(base), uint64_t(dim), uint64_t(n_states), uint64_t(c0), nc);
+                launch_columns<T, 1, true>(const_cast<V *>(static_cast<V const *>(states)),
+                                           reinterpret_cast<V *>(base), dim, n_states, c0, nc, st);
                 FP_LAUNCHED();
                 cols = reinterpret_cast<P const *>(base);
             }
             uint32_t const groups = (nc + g.per_group - 1) / g.per_group;
-            uint64_t const blocks = uint64_t(n_items) * (xcd ? (groups + 7) / 8 * 8 : groups);
+            uint64_t const blocks = uint64_t(n_items) * groups;
             hipLaunchKernelGGL(fpc::k_ev_columns<T>, dim3(uint32_t(blocks)), dim3(fpc::kThreads), fpc::kTileBytes, st,
-                               cols, uint32_t(ops->n_qubits), nc, n_items, groups, xcd ? 1 : 0,
+                               cols, uint32_t(ops->n_qubits), nc, n_items, groups,
                                reinterpret_cast<fpc::ColItem const *>(d_tables),
                                reinterpret_cast<fpc::ColEntry const *>(d_tables + tt->o_chunks),
                                reinterpret_cast<fpc::ColStr const *>(d_tables + tt->o_strs), partial);
@@ -205,7 +211,224 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
     return s;
 }
 
+// ---------------------------------------------------------------------------
+// Apply on columns
+// ---------------------------------------------------------------------------
+
+namespace
+{
+
+// Configurations of k_apply_columns: one row a thread and four strings in flight, straight from
+// the column; or 2^13-row tiles in LDS, eight rows a thread.
+template <class T, int NS, bool WTD>
+fp_status launch_apply_columns(void const *cols, void *out, uint32_t n, uint32_t n_cols, uint32_t n_states,
+                               fpc::XZ const *xz, T const *cf, uint64_t cf_stride, uint32_t n_strings, uint32_t shift,
+                               int accumulate, bool lds, hipStream_t st)
+{
+    typedef typename fpk::VecOf<T, NS>::type V;
+    auto go = [&](auto e_tag, auto u_tag, auto th_tag, auto lds_tag) -> fp_status {
+        constexpr int E = decltype(e_tag)::value, U = decltype(u_tag)::value, TH = decltype(th_tag)::value;
+        constexpr bool LDS = decltype(lds_tag)::value;
+        constexpr uint32_t kTile = 6u + fpc::log2c(E) + fpc::log2c(TH / 64);
+        constexpr size_t kLds = LDS ? sizeof(V) * E * TH : 0;
+        auto const kfn = &fpc::k_apply_columns<T, NS, E, U, TH, LDS, !LDS, WTD>;
+        if constexpr (LDS)
+        {
+            static std::once_flag once;
+            static hipError_t attr = hipSuccess;
+            std::call_once(once, [&] {
+                attr = hipFuncSetAttribute(reinterpret_cast<void const *>(kfn),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
+            });
+            if (attr != hipSuccess)
+                return fail(FP_ERR_RUNTIME, "hipFuncSetAttribute failed: %s", hipGetErrorString(attr));
+        }
+        uint32_t const tiles = n > kTile ? 1u << (n - kTile) : 1u, per = n < kTile ? 1u << (kTile - n) : 1u;
+        uint32_t const groups = (n_cols + per - 1) / per;
+        hipLaunchKernelGGL(kfn, dim3(tiles * groups), dim3(TH), kLds, st, static_cast<V const *>(cols),
+                           static_cast<V *>(out), n, n_cols, groups, tiles, xz, cf, cf_stride, n_states, n_strings,
+                           shift, accumulate);
+        FP_LAUNCHED();
+        return FP_OK;
+    };
+    typedef std::integral_constant<int, 1> I1;
+    typedef std::integral_constant<int, 4> I4;
+    typedef std::integral_constant<int, 8> I8;
+    typedef std::integral_constant<int, 256> I256;
+    typedef std::integral_constant<int, 1024> I1024;
+    return lds ? go(I8{}, I1{}, I1024{}, std::true_type{}) : go(I1{}, I4{}, I256{}, std::false_type{});
+}
+
+// The LDS tiles: columns of 2^9 to 2^14 rows, most of whose partner rows they hold, when the
+// tiles fill the chip; and columns as large as an XCD's L2 (2^18 rows of 16 bytes).
+bool apply_lds_tiles(uint32_t n, uint64_t n_cols)
+{
+    uint64_t const tiles = n > 13 ? n_cols << (n - 13) : n_cols >> (13 - n);
+    return n >= 9 && (n <= 14 || n == 18) && tiles >= 192 && lds_bytes() >= (size_t(1) << 17);
+}
+
+} // namespace
+
+// How an apply runs: 0 on the row-major batch (streaming or coset-tiled kernels), 1 as one
+// column made of the whole batch, 2 on transposed columns.
+//  1: a power-of-two state count (weighted: one state, whose weights are then one row) and a
+//     batch of at most 8 MiB (one state: 32 MiB), which the L2s and the Infinity Cache serve;
+//     beyond 4 MiB from 64 strings (n = 20, one complex128 state: N = 24 41.6 us streaming /
+//     45.9, N = 64 113 / 112).  us, streaming / column: n = 10, 128 states, 64 strings 14.1 / 7.4;
+//     n = 18, one state, 1000 strings 286 / 148.
+//  2: columns of at most 4 MiB (an XCD's L2), 8 MiB where the state count is not a power of two
+//     (the coset-tiled kernel is then at its slowest); enough work to pay the two transposed
+//     copies: from 32 strings and 3e7 (string, element) terms.  us, streaming or tiled / columns:
+//     n = 14, 1000 complex128 states, 500 strings 8500 / 3270; n = 20, 19 complex64 states, 512
+//     strings 10900 / 5710; but n = 12, 100 complex64 states, 64 strings (2.6e7 terms) 16.2 / 21.3
+//     and n = 20, 16 complex64 states, 64 strings 619 / 733.
+// FAST_PAULI_APPLY_KERNEL=columns forces 1 or 2 where the shape allows, other values forbid them.
+int apply_columns_route(fp_hip_ops const *ops, int dtype, size_t n_states, bool weighted)
+{
+    size_t const n = ops->n_qubits, N = ops->n_strings, esz = dtype == FP_C128 ? 16 : 8;
+    if (N < 2 || n > 24 || n_states > (size_t(1) << 24))
+        return 0;
+    char const *v = std::getenv("FAST_PAULI_APPLY_KERNEL");
+    bool const forced = v && std::strcmp(v, "columns") == 0;
+    if (v && *v && !forced)
+        return 0;
+    size_t const elements = (size_t(1) << n) * n_states;
+    bool const pow2 = (n_states & (n_states - 1)) == 0;
+    if (pow2 && (!weighted || n_states == 1) && elements >= 64 &&
+        elements * esz <= (n_states == 1 ? size_t(32) << 20 : size_t(8) << 20) &&
+        (elements * esz <= (size_t(4) << 20) || N >= 64 || forced))
+        return 1;
+    size_t const col_bytes = (size_t(1) << n) * esz;
+    if (n < 6 || col_bytes > (size_t(8) << 20))
+        return 0;
+    if (forced)
+        return 2;
+    if (col_bytes > (size_t(4) << 20) && pow2)
+        return 0;
+    return N >= 32 && double(N) * double(elements) >= 3e7 ? 2 : 0;
+}
+
+fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void const *states, void const *data,
+                            void *out, size_t dim, size_t n_states, int accumulate, hipStream_t st, bool *done)
+{
+    *done = false;
+    bool const weighted = kind == kTilesWeightedApply, c64 = dtype != FP_C128;
+    int const route = apply_columns_route(ops, dtype, n_states, weighted);
+    if (route == 0 || (route == 2 || weighted ? capturing(st) : false))
+        return FP_OK;
+    uint32_t const n = uint32_t(ops->n_qubits), N = uint32_t(ops->n_strings);
+    size_t const esz = c64 ? 8 : 16;
+    auto const *xz = ops->d_xz;
+    bool const aligned16 = ((reinterpret_cast<uintptr_t>(states) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
+    // scratch: [transposed states | transposed outputs | weights]
+    bool const pairs = c64 && n <= 18 && n_states > 1;
+    uint32_t const ns = pairs ? 2u : 1u;
+    size_t const col_bytes = dim * esz * ns;
+    size_t const all_cols = (n_states + ns - 1) / ns;
+    size_t cols = route == 2 ? std::max<size_t>(1, std::min(kSlabBytes / col_bytes, all_cols)) : 0;
+    if (cols < all_cols && cols >= 8)
+        cols = cols / 8 * 8; // as many columns on every XCD
+    size_t const slab = round256(cols * col_bytes);
+    size_t const w_bytes = weighted ? round256(n_states * size_t(N) * esz + fpc::kXzPad * esz) : 0;
+    unsigned char *base = nullptr;
+    std::unique_ptr<StreamGuard> guard; // held until the kernels that use the scratch are enqueued
+    if (2 * slab + w_bytes > 0)
+    {
+        guard = std::make_unique<StreamGuard>(st);
+        void *scratch = nullptr;
+        fp_status const s = scratch_get(st, 2 * slab + w_bytes, &scratch);
+        if (s == FP_ERR_OUT_OF_MEMORY)
+        {
+            (void)hipGetLastError();
+            return FP_OK; // no room: the kernels that read the batch as it is
+        }
+        if (s != FP_OK)
+            return s;
+        base = static_cast<unsigned char *>(scratch);
+    }
+    auto run = [&](auto T_tag, auto const *coef) -> fp_status {
+        typedef decltype(T_tag) T;
+        typedef typename fpk::VecOf<T, 1>::type V1;
+        T *w = nullptr;
+        if (weighted)
+        {
+            w = reinterpret_cast<T *>(base + 2 * slab);
+            constexpr int R = 8;
+            dim3 const grid(uint32_t((n_states + 255) / 256), (N + R - 1) / R);
+            hipLaunchKernelGGL((fpc::k_weights<T, R>), grid, dim3(256), 0, st, coef, static_cast<T const *>(data),
+                               ops->d_ny, w, uint64_t(N), uint64_t(ops->n_operators), uint64_t(n_states));
+            FP_LAUNCHED();
+        }
+        if (route == 1)
+        {
+            uint32_t shift = 0;
+            while ((size_t(1) << shift) < n_states)
+                ++shift;
+            // complex64: two states a row where that leaves enough waves
+            bool const two = c64 && shift > 0 && aligned16 && dim * n_states >= (size_t(1) << 19);
+            if constexpr (sizeof(T) == 4)
+                if (two)
+                    return launch_apply_columns<T, 2, false>(states, out, n + shift - 1, 1, 1, xz, coef, 0, N,
+                                                             shift - 1, accumulate, false, st);
+            return weighted ? launch_apply_columns<T, 1, true>(states, out, n, 1, 1, xz, w, N, N, 0, accumulate, false, st)
+                            : launch_apply_columns<T, 1, false>(states, out, n + shift, 1, 1, xz, coef, 0, N, shift,
+                                                                accumulate, false, st);
+        }
+        auto slabs = [&](auto ns_tag) -> fp_status {
+            constexpr int NS = decltype(ns_tag)::value;
+            typedef typename fpk::VecOf<T, NS>::type V;
+            auto *ic = reinterpret_cast<V *>(base), *oc = reinterpret_cast<V *>(base + slab);
+            for (size_t c0 = 0; c0 < n_states; c0 += cols * NS)
+            {
+                uint32_t const nst = uint32_t(std::min<size_t>(cols * NS, n_states - c0));
+                uint32_t const nc = (nst + NS - 1) / NS;
+                launch_columns<T, NS, true>(const_cast<V1 *>(static_cast<V1 const *>(states)), ic, dim, n_states, c0,
+                                            nst, st);
+                if (accumulate)
+                    launch_columns<T, NS, true>(static_cast<V1 *>(out), oc, dim, n_states, c0, nst, st);
+                FP_LAUNCHED();
+                bool const lds = apply_lds_tiles(n, nc);
+                fp_status const s =
+                    weighted ? launch_apply_columns<T, NS, true>(ic, oc, n, nc, nst, xz, w + 2 * c0 * N, N, N, 0,
+                                                                 accumulate, lds, st)
+                             : launch_apply_columns<T, NS, false>(ic, oc, n, nc, nst, xz, coef, 0, N, 0, accumulate,
+                                                                  lds, st);
+                if (s != FP_OK)
+                    return s;
+                launch_columns<T, NS, false>(static_cast<V1 *>(out), oc, dim, n_states, c0, nst, st);
+                FP_LAUNCHED();
+            }
+            return FP_OK;
+        };
+        if constexpr (sizeof(T) == 4)
+            if (pairs)
+                return slabs(std::integral_constant<int, 2>{});
+        return slabs(std::integral_constant<int, 1>{});
+    };
+    fp_status s;
+    if (dtype == FP_C128)
+        s = run(double{}, weighted ? ops->d_h128 : kind == kTilesSummedApply ? ops->d_rowsum128 : ops->d_cf128);
+    else
+        s = run(float{}, weighted ? ops->d_h64 : kind == kTilesSummedApply ? ops->d_rowsum64 : ops->d_cf64);
+    *done = s == FP_OK;
+    return s;
+}
+
 } // namespace fprt
+
+extern "C" fp_status fp_hip_op_apply_columns(fp_hip_ops const *ops, int dtype, size_t dim, size_t n_states, int weighted,
+                                             int *columns)
+{
+    if (!ops || !columns)
+        return fail(FP_ERR_INVALID_ARGUMENT, "NULL ops or result");
+    if (dtype != FP_C128 && dtype != FP_C64)
+        return fail(FP_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);
+    if (n_states == 0 || dim != (size_t(1) << ops->n_qubits))
+        return fail(FP_ERR_INVALID_ARGUMENT, "shape (%zu, %zu) does not match %zu qubits", dim, n_states,
+                    ops->n_qubits);
+    *columns = fprt::apply_columns_route(ops, dtype, n_states, weighted != 0) != 0 ? 1 : 0;
+    return FP_OK;
+}
 
 extern "C" fp_status fp_hip_op_expectation_columns(fp_hip_ops const *ops, int dtype, size_t dim, size_t n_states,
                                                    int *columns)

@@ -67,6 +67,25 @@ __device__ __forceinline__ void load_partners(typename Piece<T>::type (&R)[8], u
             R[i] = *reinterpret_cast<typename Piece<T>::type const *>(part + ((i ^ XS) << 10));
 }
 
+// Block `b` of per_group blocks for each of n_groups column groups.  Block ids are dealt to the
+// 8 XCDs round-robin: the blocks of a group follow each other on one XCD, whose L2 then serves
+// the columns' repeated reads; the last n_groups % 8 groups are spread over all of them.
+struct BlockOf
+{
+    uint32_t group, index;
+};
+__device__ __forceinline__ BlockOf block_of(uint32_t b, uint32_t per_group, uint32_t n_groups)
+{
+    uint32_t const whole = n_groups & ~7u;
+    if (b < whole * per_group)
+    {
+        uint32_t const slot = b >> 3;
+        return BlockOf{(slot / per_group) * 8u + (b & 7u), slot % per_group};
+    }
+    uint32_t const r = b - whole * per_group;
+    return BlockOf{whole + r / per_group, r % per_group};
+}
+
 // One string on the leader slots L and their partners R.  sg[k]: sign factor of slot bit k,
 // s0: of the sub bit.
 template <class T, int XS, bool SUB, bool IM, bool HALF>
@@ -125,12 +144,12 @@ __device__ __forceinline__ T self_sum(typename Piece<T>::type const (&L)[8], T c
     return v[0];
 }
 
-// cols: n_cols columns of 2^n rows, back to back.  Block b runs item `b % n_items` (or, with
-// xcd != 0, the items of one column on one XCD) on column tile group `y`: one column, or the
-// 2^(tile_bits - n) columns that fill a tile.  partial[item * n_cols + t]: FP64 sums.
+// cols: n_cols columns of 2^n rows, back to back.  A block runs one item on one column group:
+// one column, or the 2^(tile_bits - n) columns that fill a tile.  partial[item * n_cols + t]:
+// FP64 sums.
 template <class T>
 __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::type const *__restrict__ cols, uint32_t n,
-                                                         uint32_t n_cols, uint32_t n_items, uint32_t n_groups, int xcd,
+                                                         uint32_t n_cols, uint32_t n_items, uint32_t n_groups,
                                                          ColItem const *__restrict__ items,
                                                          ColEntry const *__restrict__ entries,
                                                          ColStr const *__restrict__ strs,
@@ -143,22 +162,8 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
     P *tile = reinterpret_cast<P *>(smem);
     __shared__ double red[2][kThreads / 64];
 
-    uint32_t grp, it;
-    if (xcd)
-    {
-        // block ids are dealt to the 8 XCDs round-robin: the items of one column group follow
-        // each other on one XCD, whose L2 keeps the column
-        uint32_t const slot = blockIdx.x >> 3;
-        grp = (slot / n_items) * 8u + (blockIdx.x & 7u);
-        it = slot % n_items;
-        if (grp >= n_groups)
-            return;
-    }
-    else
-    {
-        grp = blockIdx.x / n_items;
-        it = blockIdx.x % n_items;
-    }
+    BlockOf const bo = block_of(blockIdx.x, n_items, n_groups);
+    uint32_t const grp = bo.group, it = bo.index;
     ColItem const item = items[it];
     uint32_t const tid = threadIdx.x, lane = tid & 63u;
     uint32_t const wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -346,25 +351,68 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
     }
 }
 
-// Columns [c0, c0 + n_cols) of a row-major (rows x ld) batch, each made contiguous:
-// out[c * rows + r] = in[r * ld + c0 + c].  32 x 32 tiles through LDS.
-template <class V>
-__global__ __launch_bounds__(256) void k_columns_in(V const *__restrict__ in, V *__restrict__ out, uint64_t rows,
-                                                    uint64_t ld, uint64_t c0, uint32_t n_cols)
+// Columns [c0, c0 + n_cols) of a row-major (rows x ld) batch to columns of NS states a row, and
+// back (IN = false).  Tiles of 32 rows x 32 states through LDS; an odd last state is paired with
+// zeros, which are not written back.
+template <class T, int NS, bool IN>
+__global__ __launch_bounds__(256) void k_columns(typename fpk::VecOf<T, 1>::type *__restrict__ batch,
+                                                 typename fpk::VecOf<T, NS>::type *__restrict__ cols, uint64_t rows,
+                                                 uint64_t ld, uint64_t c0, uint32_t n_cols)
 {
-    __shared__ V tile[32][33];
+    typedef typename fpk::VecOf<T, 1>::type V1;
+    typedef typename fpk::VecOf<T, NS>::type V;
+    __shared__ V1 tile[32][33];
     uint64_t const r0 = uint64_t(blockIdx.x) * 32;
     uint32_t const cb = blockIdx.y * 32u;
     uint32_t const tx = threadIdx.x & 31u, ty = threadIdx.x >> 5;
+    auto batch_side = [&] {
 #pragma unroll
-    for (uint32_t k = ty; k < 32; k += 8)
-        if (r0 + k < rows && cb + tx < n_cols)
-            tile[k][tx] = in[(r0 + k) * ld + c0 + cb + tx];
+        for (uint32_t k = ty; k < 32; k += 8)
+            if (r0 + k < rows)
+            {
+                V1 *at = batch + (r0 + k) * ld + c0 + cb + tx;
+                bool const live = cb + tx < n_cols;
+                if constexpr (IN)
+                    tile[k][tx] = live ? *at : V1(0);
+                else if (live)
+                    __builtin_nontemporal_store(tile[k][tx], at);
+            }
+    };
+    auto column_side = [&] {
+#pragma unroll
+        for (uint32_t k = ty; k < 32 / NS; k += 8)
+            if (r0 + tx < rows && cb + k * NS < n_cols)
+            {
+                V *at = cols + uint64_t(cb / NS + k) * rows + r0 + tx;
+                if constexpr (IN)
+                {
+                    V v;
+#pragma unroll
+                    for (int h = 0; h < NS; ++h)
+                    {
+                        v[2 * h] = tile[tx][k * NS + h][0];
+                        v[2 * h + 1] = tile[tx][k * NS + h][1];
+                    }
+                    *at = v;
+                }
+                else
+                {
+                    V const v = *at;
+#pragma unroll
+                    for (int h = 0; h < NS; ++h)
+                        tile[tx][k * NS + h] = V1{v[2 * h], v[2 * h + 1]};
+                }
+            }
+    };
+    if constexpr (IN)
+        batch_side();
+    else
+        column_side();
     __syncthreads();
-#pragma unroll
-    for (uint32_t k = ty; k < 32; k += 8)
-        if (r0 + tx < rows && cb + k < n_cols)
-            out[uint64_t(cb + k) * rows + r0 + tx] = tile[tx][k];
+    if constexpr (IN)
+        column_side();
+    else
+        batch_side();
 }
 
 } // namespace fpc

@@ -141,6 +141,7 @@ void free_device(fp_hip_ops *o)
     o->d_arena = nullptr;
     o->arena_bytes = 0;
     o->d_x = o->d_z = nullptr;
+    o->d_xz = nullptr;
     o->d_meta = nullptr;
     o->d_ny = nullptr;
     o->d_cf128 = o->d_scale = o->d_kappa_c = o->d_kappa = o->d_rowsum128 = o->d_wr64 = o->d_wi64 = nullptr;
@@ -194,20 +195,21 @@ double kappa_of(uint64_t x, uint32_t ny)
     return ((ny & 3u) == 1u) ? 2.0 : -2.0;
 }
 
+// (padded: the apply kernel on columns reads past the end of the row sums)
 template <class T> fp_status upload(T **dptr, std::vector<T> const &h)
 {
     if (*dptr == nullptr)
-        FP_HIP(hipMalloc(reinterpret_cast<void **>(dptr), std::max<size_t>(h.size(), 1) * sizeof(T)));
+        FP_HIP(hipMalloc(reinterpret_cast<void **>(dptr), (h.size() + 2 * fpc::kXzPad) * sizeof(T)));
     if (!h.empty())
         FP_HIP(hipMemcpy(*dptr, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
     return FP_OK;
 }
 
-// Arena layout: x | z | ny | meta | cf128 | cf64 | scale | kappa_c | kappa,
+// Arena layout: xz | x | z | ny | meta | cf128 | cf64 | scale | kappa_c | kappa,
 // each section 256-byte aligned.
 struct ArenaLayout
 {
-    size_t x, z, ny, meta, cf128, cf64, scale, kappa_c, kappa, ev_chunks, ev_strs, total;
+    size_t xz, x, z, ny, meta, cf128, cf64, scale, kappa_c, kappa, ev_chunks, ev_strs, total;
 };
 
 ArenaLayout arena_layout(size_t N)
@@ -215,12 +217,14 @@ ArenaLayout arena_layout(size_t N)
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     ArenaLayout L{};
     size_t off = 0;
+    // (the apply kernel on columns reads kXzPad records past the end of xz, cf128 and cf64)
+    L.xz = off, off += up((N + fpc::kXzPad) * sizeof(fpc::XZ));
     L.x = off, off += up(N * sizeof(uint64_t));
     L.z = off, off += up(N * sizeof(uint64_t));
     L.ny = off, off += up(N * sizeof(uint32_t));
     L.meta = off, off += up(N * sizeof(fpk::StringMeta));
-    L.cf128 = off, off += up(2 * N * sizeof(double));
-    L.cf64 = off, off += up(2 * N * sizeof(float));
+    L.cf128 = off, off += up(2 * (N + fpc::kXzPad) * sizeof(double));
+    L.cf64 = off, off += up(2 * (N + fpc::kXzPad) * sizeof(float));
     L.scale = off, off += up(2 * N * sizeof(double));
     L.kappa_c = off, off += up(2 * N * sizeof(double));
     L.kappa = off, off += up(N * sizeof(double));
@@ -386,6 +390,7 @@ fp_status ops_assign(fp_hip_ops *o, size_t n_qubits, size_t n_strings, uint8_t c
         o->ny[s] = ny;
         uint32_t const hb = x ? 63u - uint32_t(__builtin_clzll(x)) : 0u;
         uint32_t const mode = x == 0 ? fpk::kModeSelf : ((ny & 1u) ? fpk::kModeIm : fpk::kModeRe);
+        at<fpc::XZ>(h, L.xz)[s] = fpc::XZ{uint32_t(x), uint32_t(z)};
         at<uint64_t>(h, L.x)[s] = x;
         at<uint64_t>(h, L.z)[s] = z;
         at<uint32_t>(h, L.ny)[s] = ny;
@@ -408,6 +413,7 @@ fp_status ops_assign(fp_hip_ops *o, size_t n_qubits, size_t n_strings, uint8_t c
         o->arena_bytes = L.total;
     }
     void *d = o->d_arena;
+    o->d_xz = at<fpc::XZ>(d, L.xz);
     o->d_x = at<uint64_t>(d, L.x);
     o->d_z = at<uint64_t>(d, L.z);
     o->d_ny = at<uint32_t>(d, L.ny);
@@ -1329,6 +1335,11 @@ fp_status fp_hip_op_apply(fp_hip_ops const *ops, int dtype, void const *states, 
     if ((st = check_no_alias(dtype, states, out, dim, n_states)) != FP_OK)
         return st;
     hipStream_t const s = static_cast<hipStream_t>(stream);
+    bool done = false;
+    st = fprt::run_apply_columns(ops, dtype, fprt::kTilesOpApply, states, nullptr, out, dim, n_states, accumulate, s,
+                                 &done);
+    if (st != FP_OK || done)
+        return st;
     bool tiled = false;
     if ((st = fprt::choose_op_apply_tiled(ops, dtype, n_states, &tiled)) != FP_OK)
         return st;
@@ -1478,6 +1489,11 @@ fp_status fp_hip_summed_apply(fp_hip_ops const *ops, int dtype, void const *stat
     if ((st = check_no_alias(dtype, states, out, dim, n_states)) != FP_OK)
         return st;
     hipStream_t const s = static_cast<hipStream_t>(stream);
+    bool done = false;
+    st = fprt::run_apply_columns(ops, dtype, fprt::kTilesSummedApply, states, nullptr, out, dim, n_states, accumulate,
+                                 s, &done);
+    if (st != FP_OK || done)
+        return st;
     // large states whose strings share coset tiles: the tiled kernel (same operations, same order)
     bool use_tiled = false;
     if ((st = fprt::choose_op_apply_tiled(ops, dtype, n_states, &use_tiled, fprt::kTilesSummedApply)) != FP_OK)
@@ -1514,6 +1530,11 @@ fp_status fp_hip_summed_apply_weighted(fp_hip_ops const *ops, int dtype, void co
         return fail(FP_ERR_INVALID_ARGUMENT, "out must not overlap data");
     hipStream_t const s = static_cast<hipStream_t>(stream);
     StreamGuard guard(s);
+    bool done = false;
+    st = fprt::run_apply_columns(ops, dtype, fprt::kTilesWeightedApply, states, data, out, dim, n_states, accumulate, s,
+                                 &done);
+    if (st != FP_OK || done)
+        return st;
     size_t const N = ops->n_strings, K = ops->n_operators, S = n_states;
     size_t const esz = dtype == FP_C128 ? sizeof(double) : sizeof(float);
     void *scratch = nullptr;

@@ -15,6 +15,7 @@
 
 #include "fast_pauli_hip.h"
 #include "fp_ev_lds.hpp"
+#include "fp_apply_columns.hpp"
 #include "fp_apply_tiled.hpp"
 #include "fp_ev_tiled.hpp"
 #include "fp_kernels.hpp"
@@ -191,6 +192,14 @@ fp_status run_op_expect(fp_hip_ops const *ops, int dtype, void const *states, vo
 bool ev_columns_eligible(fp_hip_ops const *ops, int dtype, size_t n_states);
 fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *states, void *out, size_t dim,
                                 size_t n_states, int accumulate, hipStream_t st, Workspace const *ws, bool *done);
+// Apply on columns (fp_apply_columns.hpp), for the kinds kTilesOpApply, kTilesSummedApply and
+// kTilesWeightedApply (`data`: the real (operators x states) weights).  *done = false, with
+// nothing enqueued, when the shape runs on the row-major kernels, or there is no room for the
+// transposed slabs, or they would be needed while the stream is being captured.  Holds the
+// stream's StreamGuard while it uses its scratch.
+int apply_columns_route(fp_hip_ops const *ops, int dtype, size_t n_states, bool weighted);
+fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void const *states, void const *data,
+                            void *out, size_t dim, size_t n_states, int accumulate, hipStream_t st, bool *done);
 // Shape checks shared by the entry points.
 fp_status check_shape(fp_hip_ops const *ops, int dtype, void const *a, void const *b, size_t dim, size_t n_states);
 // Sets up the allocation-free entry point's static buffer on the current device
@@ -241,6 +250,7 @@ struct fp_hip_ops
     // device copies (pointers into the arena)
     uint64_t *d_x = nullptr, *d_z = nullptr;
     fpk::StringMeta *d_meta = nullptr;
+    fpc::XZ *d_xz = nullptr;     // x and z in 32 bits (n <= 32), read kXzPad records past the end
     double *d_cf128 = nullptr;   // c_s * (-i)^{nY_s}, complex128
     float *d_cf64 = nullptr;     // same, complex64
     double *d_scale = nullptr;   // c_s * kappa_s (complex, FP64): PauliOp EV

@@ -234,5 +234,11 @@ struct ColStr
     double sim;
 };
 
+// One string's masks (n <= 32), for the apply kernel on columns.
+struct XZ
+{
+    uint32_t x, z;
+};
+
 } // namespace fpc
 

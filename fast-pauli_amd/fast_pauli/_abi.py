@@ -87,6 +87,7 @@ _SIGS = {
     "fp_hip_op_expectation": [_vp, _i, _vp, _vp, _sz, _sz, _i, _vp],
     "fp_hip_op_expectation_plan": [_vp, _i, _sz, _sz, _vp],
     "fp_hip_op_expectation_columns": [_vp, _i, _sz, _sz, ctypes.POINTER(_i)],
+    "fp_hip_op_apply_columns": [_vp, _i, _sz, _sz, _i, ctypes.POINTER(_i)],
     "fp_hip_op_apply_plan": [_vp, _i, _sz, _sz, _i, _vp],
     "fp_hip_summed_apply_plan": [_vp, _i, _sz, _sz, _i, _vp],
     "fp_hip_summed_apply_weighted_plan": [_vp, _i, _sz, _sz, _i, _vp],
@@ -124,6 +125,13 @@ def op_expectation_columns(ops, dtype: int, dim: int, n_states: int) -> bool:
     return bool(c.value)
 
 
+def op_apply_columns(ops, dtype: int, dim: int, n_states: int, weighted: bool = False) -> bool:
+    """Whether fp_hip_op_apply and its SummedPauliOp forms run these shapes on columns."""
+    c = _i(0)
+    call("fp_hip_op_apply_columns", ops.handle, dtype, dim, n_states, int(bool(weighted)), ctypes.byref(c))
+    return bool(c.value)
+
+
 def op_expectation_plan(ops, dtype: int, dim: int, n_states: int) -> dict:
     """The row-major kernel of fp_hip_op_expectation for these shapes, and its HBM bytes."""
     p = EvPlan()
@@ -132,7 +140,7 @@ def op_expectation_plan(ops, dtype: int, dim: int, n_states: int) -> dict:
 
 
 def op_apply_plan(ops, dtype: int, dim: int, n_states: int, accumulate: bool = False) -> dict:
-    """Which kernel fp_hip_op_apply runs for these shapes, and its HBM bytes."""
+    """The row-major kernel of fp_hip_op_apply for these shapes, and its HBM bytes."""
     p = EvPlan()
     call("fp_hip_op_apply_plan", ops.handle, dtype, dim, n_states, int(bool(accumulate)), ctypes.byref(p))
     return p.as_dict()

@@ -223,8 +223,19 @@ typedef struct fp_hip_ev_plan
 fp_status fp_hip_op_expectation_plan(fp_hip_ops const *ops, int dtype, size_t dim, size_t n_states,
                                      fp_hip_ev_plan *plan);
 
-/* Which kernel fp_hip_op_apply runs for these shapes, in the same record (no reference
- * counterpart: for measurement and triage).  kernel 0 (FP_EV_STREAM): every string reads the
+/* Whether fp_hip_op_apply and fp_hip_summed_apply (weighted != 0: fp_hip_summed_apply_weighted)
+ * run these shapes on columns: the whole batch as one column where the state count is a power of
+ * two and the batch small, else each state made one contiguous column (transposed copies of at
+ * most 128 MiB of states and as much of outputs in the stream's scratch).  No counterpart in the
+ * reference.  Results are IEEE-equal either way.  Where the copies have no room, or the stream is
+ * being captured and they would be needed, the call runs the kernel of fp_hip_op_apply_plan (or
+ * its SummedPauliOp forms) instead. */
+fp_status fp_hip_op_apply_columns(fp_hip_ops const *ops, int dtype, size_t dim, size_t n_states, int weighted,
+                                  int *columns);
+
+/* Which row-major kernel fp_hip_op_apply runs for these shapes when fp_hip_op_apply_columns does
+ * not say that it takes columns, in the same record (no reference counterpart: for measurement
+ * and triage).  kernel 0 (FP_EV_STREAM): every string reads the
  * state once and the output is written once.  kernel 1 (FP_EV_TILED): groups of consecutive
  * strings, one launch each, every group reading the state and reading and writing the output
  * (the first group does not read it unless accumulating).  hbm_bytes counts those reads and

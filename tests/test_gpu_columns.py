@@ -88,3 +88,111 @@ def test_expectation_columns_rule(hip, monkeypatch):
     assert not _abi.op_expectation_columns(ops, C128, 1 << 14, 100)
     with pytest.raises(ValueError):
         _abi.op_expectation_columns(ops, C128, 1 << 13, 100)
+
+
+# ---------------------------------------------------------------------------
+# apply: IEEE-equal to the oracle's sequential loop
+# ---------------------------------------------------------------------------
+def _odt(dtype):
+    return O.C128 if dtype == C128 else O.C64
+
+
+@pytest.mark.parametrize("dtype,n,S", [
+    # one column made of the batch (power-of-two state counts), one wave to many
+    (C128, 6, 1), (C128, 5, 2), (C128, 10, 16), (C128, 13, 1), (C64, 6, 1), (C64, 8, 4), (C64, 12, 128), (C64, 15, 1),
+    # transposed columns: shorter and longer than a block, odd counts (complex64: a state paired with zeros)
+    (C128, 6, 5), (C128, 7, 33), (C128, 9, 3), (C128, 13, 3), (C64, 6, 3), (C64, 7, 40), (C64, 10, 33), (C64, 14, 6),
+    # tiles in LDS: columns shorter than a tile (a ragged last group), of one tile and of two
+    (C128, 11, 771), (C128, 13, 193), (C128, 14, 97), (C64, 12, 771), (C64, 14, 195),
+])
+@pytest.mark.parametrize("kind", ["random", "weight2"])
+def test_apply_on_columns(hip, monkeypatch, kind, dtype, n, S):
+    H.say(f"apply on columns {kind} n={n} S={S} dtype={dtype}")
+    monkeypatch.setenv("FAST_PAULI_APPLY_KERNEL", "columns")
+    cdt = H.CDT[dtype]
+    codes = _structured_codes(kind, 29, n, seed=n + S)
+    strings = syn.codes_to_strings(codes)
+    coeffs = syn.random_coeffs(29, seed=S + 2)
+    ops = _abi.Ops(codes, coeffs)
+    assert _abi.op_apply_columns(ops, dtype, 1 << n, S)
+    psi = syn.random_states(1 << n, S, seed=n * 17 + S).astype(cdt)
+    got = H.op_apply(ops, psi, dtype)
+    assert np.array_equal(got, O.op_apply(strings, coeffs.astype(cdt), psi, np.zeros_like(psi), dtype=_odt(dtype)))
+    base = syn.random_states(1 << n, S, seed=n + 12).astype(cdt)
+    got = H.op_apply(ops, psi, dtype, out0=base)
+    assert np.array_equal(got, O.op_apply(strings, coeffs.astype(cdt), psi, base.copy(), dtype=_odt(dtype)))
+
+
+@pytest.mark.parametrize("N", [2, 3, 4, 5, 7, 8, 23, 24, 25, 48])
+def test_apply_on_columns_string_counts(hip, monkeypatch, N):
+    """Every remainder of the strings in flight and of the unrolled stages."""
+    H.say(f"apply on columns N={N}")
+    monkeypatch.setenv("FAST_PAULI_APPLY_KERNEL", "columns")
+    for n, S in ((9, 4), (13, 200)):
+        codes, coeffs = syn.random_codes(N, n, seed=N), syn.random_coeffs(N, seed=N)
+        psi = syn.random_states(1 << n, S, seed=N + n)
+        got = H.op_apply(_abi.Ops(codes, coeffs), psi, C128)
+        assert np.array_equal(got, O.op_apply(syn.codes_to_strings(codes), coeffs, psi, np.zeros_like(psi)))
+
+
+@pytest.mark.parametrize("dtype,n,N,K,S", [(C128, 8, 40, 3, 5), (C128, 14, 33, 9, 97), (C64, 9, 50, 7, 37),
+                                           (C64, 14, 20, 4, 195), (C128, 12, 30, 5, 1), (C64, 11, 17, 300, 1)])
+def test_summed_apply_on_columns(hip, monkeypatch, dtype, n, N, K, S):
+    """SummedPauliOp::apply and apply_weighted (per-state weights), overwrite and accumulate."""
+    H.say(f"summed apply on columns n={n} N={N} K={K} S={S} dtype={dtype}")
+    monkeypatch.setenv("FAST_PAULI_APPLY_KERNEL", "columns")
+    cdt = H.CDT[dtype]
+    codes = syn.random_codes(N, n, seed=n * 5 + N)
+    strings = syn.codes_to_strings(codes)
+    rng = np.random.default_rng(n + N + K + S)
+    coeffs_nk = rng.standard_normal((N, K)) + 1j * rng.standard_normal((N, K))
+    ops = _abi.Ops(codes, matrix=coeffs_nk)
+    psi = syn.random_states(1 << n, S, seed=n + S).astype(cdt)
+    data = rng.standard_normal((K, S)).astype(np.float64 if dtype == C128 else np.float32)
+    dim = 1 << n
+    assert _abi.op_apply_columns(ops, dtype, dim, S) and _abi.op_apply_columns(ops, dtype, dim, S, weighted=True)
+    d_in, d_data = _abi.DeviceBuffer.from_array(psi), _abi.DeviceBuffer.from_array(data)
+    c_dt = coeffs_nk.astype(cdt)
+    for base in (np.zeros_like(psi), syn.random_states(dim, S, seed=98).astype(cdt)):
+        acc = int(base.any())
+        d_out = _abi.DeviceBuffer.from_array(base)
+        _abi.call("fp_hip_summed_apply", ops.handle, dtype, d_in.ptr, d_out.ptr, dim, S, acc, None)
+        exp = O.summed_apply(strings, c_dt, psi, base.copy(), dtype=_odt(dtype))
+        assert np.array_equal(d_out.to_array(cdt, psi.shape), exp)
+        d_out.upload(base)
+        _abi.call("fp_hip_summed_apply_weighted", ops.handle, dtype, d_in.ptr, d_data.ptr, d_out.ptr, dim, S, acc,
+                  None)
+        exp = O.summed_apply_weighted(strings, c_dt, psi, data, base.copy(), dtype=_odt(dtype))
+        assert np.array_equal(d_out.to_array(cdt, psi.shape), exp)
+
+
+def test_apply_on_columns_several_slabs_and_unaligned(hip, monkeypatch):
+    """70 complex128 columns of 2 MiB (more than one 128 MiB slab), and complex64 buffers at 8
+    bytes past a 16-byte boundary: equal to the streaming kernel, itself checked against the oracle."""
+    H.say("apply on columns, several slabs and unaligned buffers")
+    for dtype, n, S, off in ((C128, 17, 70, 0), (C64, 12, 64, 8), (C64, 12, 33, 8), (C64, 18, 3, 0)):
+        cdt = H.CDT[dtype]
+        ops = _abi.Ops(syn.random_codes(9, n, seed=n), syn.random_coeffs(9, seed=n))
+        nbytes = (1 << n) * S * np.dtype(cdt).itemsize
+        d_in, d_out = _abi.DeviceBuffer(nbytes + 16), _abi.DeviceBuffer(nbytes + 16)
+        d_in.zero()
+        d_in.upload(np.ascontiguousarray(syn.random_states(1 << n, S, seed=n).astype(cdt)))
+        got = []
+        for kernel in ("columns", "stream"):
+            monkeypatch.setenv("FAST_PAULI_APPLY_KERNEL", kernel)
+            d_out.zero()
+            # the last state's end is outside the uploaded array when shifted: still inside the buffer
+            _abi.call("fp_hip_op_apply", ops.handle, dtype, d_in.ptr + off, d_out.ptr + off, 1 << n, S, 0, None)
+            got.append(d_out.to_array(np.uint8, (nbytes + 16,)).copy())
+        assert np.array_equal(got[0], got[1]), (dtype, n, S, off)
+
+
+def test_apply_columns_rule(hip, monkeypatch):
+    """Which shapes run on columns; the rest, and the other kernels when forced, do not."""
+    H.say("apply columns rule")
+    for n, N, S, want in ((10, 64, 128, True), (18, 1000, 1, True), (14, 500, 1000, True), (12, 64, 100, False),
+                          (20, 24, 1, False), (21, 96, 8, False), (10, 1, 128, False)):
+        ops = _abi.Ops(syn.random_codes(N, n, seed=n))
+        assert _abi.op_apply_columns(ops, C128, 1 << n, S) == want, (n, N, S)
+    monkeypatch.setenv("FAST_PAULI_APPLY_KERNEL", "tiled")
+    assert not _abi.op_apply_columns(_abi.Ops(syn.random_codes(64, 10, seed=1)), C128, 1 << 10, 128)
