@@ -83,19 +83,21 @@ constexpr uint32_t log2c(uint32_t v)
 // Records read past the last string (the tables are padded by as many).
 constexpr uint32_t kXzPad = 64;
 
-// cols, out: n_cols columns of 2^n rows; NS states a row.  A block of TH threads owns a tile of
-// TH * E rows of a column, or the columns that fill it (n_groups * tiles blocks).
+// Constant memory: uniform reads are scalar loads, also through pointers that come from a table.
+template <class P> using Const = __attribute__((address_space(4))) P const;
+
+// One block's part of an apply: group bo.group, tile bo.index of n_cols columns of 2^n rows
+// (cols to out), NS states a row.  A block of TH threads owns a tile of TH * E rows of a column,
+// or the columns that fill it.
 // LDS: the tile's rows are kept in LDS, and strings whose partner rows lie in it read them there.
 // PIPE: the next strings' partner rows are in flight while U strings are added.
 // cf: complex coefficients with (-i)^{nY} folded in; WTD: those of state t at cf + 2 * cf_stride * t.
 // shift: masks are shifted by this many bits (one column made of a whole batch).
 template <class T, int NS, int E, int U, int TH, bool LDS, bool PIPE, bool WTD>
-__global__ __launch_bounds__(TH) void k_apply_columns(typename fpk::VecOf<T, NS>::type const *__restrict__ cols,
-                                                      typename fpk::VecOf<T, NS>::type *__restrict__ out, uint32_t n,
-                                                      uint32_t n_cols, uint32_t n_groups, uint32_t tiles,
-                                                      XZ const *__restrict__ xz, T const *__restrict__ cf,
-                                                      uint64_t cf_stride, uint32_t n_states, uint32_t n_strings, uint32_t shift,
-                                                      int accumulate)
+__device__ __forceinline__ void apply_columns(BlockOf bo, typename fpk::VecOf<T, NS>::type const *__restrict__ cols,
+                                              typename fpk::VecOf<T, NS>::type *__restrict__ out, uint32_t n,
+                                              uint32_t n_cols, Const<XZ> *xz, Const<T> *cf, uint64_t cf_stride,
+                                              uint32_t n_states, uint32_t n_strings, uint32_t shift, int accumulate)
 {
     typedef typename fpk::VecOf<T, NS>::type V; // one row of NS states
     constexpr uint32_t kLe = log2c(E), kLv = log2c(sizeof(V));
@@ -105,7 +107,6 @@ __global__ __launch_bounds__(TH) void k_apply_columns(typename fpk::VecOf<T, NS>
     extern __shared__ __align__(16) unsigned char smem[];
     uint32_t const lane = threadIdx.x & 63u;
     uint32_t const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    BlockOf const bo = block_of(blockIdx.x, tiles, n_groups);
     uint32_t const grp = bo.group, p = bo.index;
     uint32_t const per = n < kTile ? 1u << (kTile - n) : 1u; // columns in a tile
     uint64_t const rows = uint64_t(1) << n;
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(TH) void k_apply_columns(typename fpk::VecOf<T, NS>
     if constexpr (LDS)
         __syncthreads();
     // WTD: the coefficients of this column's states (the last state again past the end)
-    T const *c[WTD ? NS : 1];
+    Const<T> *c[WTD ? NS : 1];
 #pragma unroll
     for (int w = 0; w < (WTD ? NS : 1); ++w)
         c[w] = cf + 2 * cf_stride * (WTD ? (tc * NS + w < n_states ? tc * NS + w : n_states - 1u) : 0u);
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(TH) void k_apply_columns(typename fpk::VecOf<T, NS>
     };
     Rec rec[3][U];
     V R[PIPE ? 2 : 1][U][E];
-    XZ const *qp = xz;
+    Const<XZ> *qp = xz;
     auto fetch = [&](int k, Rec(&r)[U]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -252,6 +253,80 @@ __global__ __launch_bounds__(TH) void k_apply_columns(typename fpk::VecOf<T, NS>
     for (int i = 0; i < E; ++i)
         if (live)
             __builtin_nontemporal_store(acc[i], oc + i * 64);
+}
+
+// One operator on n_cols columns: n_groups * tiles blocks.
+template <class T, int NS, int E, int U, int TH, bool LDS, bool PIPE, bool WTD>
+__global__ __launch_bounds__(TH) void k_apply_columns(typename fpk::VecOf<T, NS>::type const *__restrict__ cols,
+                                                      typename fpk::VecOf<T, NS>::type *__restrict__ out, uint32_t n,
+                                                      uint32_t n_cols, uint32_t n_groups, uint32_t tiles,
+                                                      XZ const *__restrict__ xz, T const *__restrict__ cf,
+                                                      uint64_t cf_stride, uint32_t n_states, uint32_t n_strings, uint32_t shift,
+                                                      int accumulate)
+{
+    apply_columns<T, NS, E, U, TH, LDS, PIPE, WTD>(block_of(blockIdx.x, tiles, n_groups), cols, out, n, n_cols,
+                                                   (Const<XZ> *)xz, (Const<T> *)cf, cf_stride, n_states, n_strings,
+                                                   shift, accumulate);
+}
+
+// Index of the first of `count` ascending ends that `pos` lies below, else >= count.  `ends` is
+// padded with its last entry to a multiple of 64: one load and a ballot for 64 of them.
+__device__ __forceinline__ uint32_t find_segment(uint32_t const *ends, uint32_t count, uint32_t pos)
+{
+    for (uint32_t base = 0; base < count; base += 64)
+    {
+        uint32_t const below = uint32_t(__popcll(__ballot(pos >= ends[base + (threadIdx.x & 63u)])));
+        if (below < 64)
+            return base + below;
+    }
+    return count;
+}
+
+// Many operators on columns of one slab (byte offsets into `in` and `out`): XCD k (blockIdx % 8)
+// works through its own n_segs segments, so the blocks of a column follow each other on one XCD
+// and every XCD gets the same number of string terms, whatever the operators' sizes.  One row a
+// thread, straight from the columns: 256 complex64 operators of n = 8..18 (3 GB of states, 5.5e10
+// terms) take 18.9 ms, 57.3 as streaming items and coset-tiled launches, 23.2 with the LDS tiles
+// for n = 9..14 and 18 (19.2 for n = 9..14, whose blocks are too few to fill their rounds).
+template <class T, int NS>
+__global__ __launch_bounds__(256) void k_apply_columns_batch(unsigned char const *__restrict__ in,
+                                                             unsigned char *__restrict__ out,
+                                                             ColJob const *__restrict__ jobs,
+                                                             uint32_t const *__restrict__ ends,
+                                                             ColSeg const *__restrict__ segs, uint32_t n_segs)
+{
+    typedef typename fpk::VecOf<T, NS>::type V;
+    constexpr uint32_t kTile = 8; // log2 rows of a block
+    uint32_t const xcd = blockIdx.x & 7u, pos = blockIdx.x >> 3;
+    uint32_t const at = __builtin_amdgcn_readfirstlane(find_segment(ends + xcd * n_segs, n_segs, pos));
+    if (at >= n_segs)
+        return;
+    ColSeg const sg = segs[xcd * n_segs + at];
+    ColJob const j = jobs[sg.job];
+    uint32_t const b = sg.block0 + (pos - sg.start);
+    uint32_t const lt = j.n > kTile ? j.n - kTile : 0u; // log2 tiles of a column
+    apply_columns<T, NS, 1, 4, 256, false, true, false>(
+        BlockOf{b >> lt, b & ((1u << lt) - 1u)}, reinterpret_cast<V const *>(in + j.cols),
+        reinterpret_cast<V *>(out + j.cols), j.n, j.n_cols, (Const<XZ> *)j.xz, (Const<T> *)j.cf, 0, 0, j.n_strings, 0,
+        int(j.accumulate));
+}
+
+// The copies of a slab's columns in (from the states, and from outputs that are added to) or out.
+template <class T, int NS, bool IN>
+__global__ __launch_bounds__(256) void k_columns_batch(unsigned char *__restrict__ in, unsigned char *__restrict__ out,
+                                                       ColCopy const *__restrict__ copies,
+                                                       uint32_t const *__restrict__ ends, uint32_t n_copies)
+{
+    typedef typename fpk::VecOf<T, 1>::type V1;
+    typedef typename fpk::VecOf<T, NS>::type V;
+    uint32_t const at = __builtin_amdgcn_readfirstlane(find_segment(ends, n_copies, blockIdx.x));
+    if (at >= n_copies)
+        return;
+    ColCopy const c = copies[at];
+    uint32_t const b = blockIdx.x - c.start, lb = c.n > 5u ? c.n - 5u : 0u; // log2 blocks of 32 rows
+    move_columns<T, NS, IN>((__attribute__((address_space(1))) V1 *)c.batch,
+                            reinterpret_cast<V *>((c.out ? out : in) + c.cols), uint64_t(1) << c.n, c.ld, c.c0,
+                            c.n_states, b & ((1u << lb) - 1u), b >> lb);
 }
 
 // w(s, t) = sum_k h(s, k) x(k, t), k in order, product then add (no contraction: the reference's

@@ -5,8 +5,10 @@
 // any qubit count, string count, state count and dtype.  The host cuts each
 // entry into work items, orders them (largest first by default), uploads the
 // descriptors, and captures [reset counters, persistent kernel] into a
-// hipGraph that is replayed on every launch.  Large apply entries whose string
-// groups share coset tiles run as coset-tiled launches of their own (one per
+// hipGraph that is replayed on every launch.  Most apply entries of a batch worth
+// it run on columns (fp_apply_columns.hpp), in rounds of many entries: three
+// launches each, after the persistent kernel in the same graph.  Of the others,
+// large apply entries whose string groups share coset tiles run as coset-tiled launches of their own (one per
 // string group, after the persistent kernel in the same graph) or become coset
 // items (one string group, a run of 64 KiB tiles each): about three state passes
 // per group instead of one per string.
@@ -74,6 +76,15 @@ struct fp_hip_batch
     };
     std::vector<Split> split;
     size_t tiled_groups = 0;
+    // entries run on columns, after those: their tables, and slabs of inputs and outputs that
+    // every round of every launch uses in turn
+    std::vector<fprt::ColumnRound> rounds;
+    size_t column_entries = 0;
+    std::vector<unsigned char> h_columns;
+    unsigned char *d_columns = nullptr, *d_slab = nullptr;
+    size_t cap_columns = 0, cap_slab = 0, slab_bytes = 0;
+    bool use_columns = true; // batch_without_columns
+    hipStream_t last_stream = nullptr;
     double plan_bytes = 0.0; // state passes of the plan: coset groups, or one per string
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -108,14 +119,16 @@ void release(fp_hip_batch *b)
     wait_idle(b);
     drop_graph(b);
     for (void *p : {static_cast<void *>(b->d_ops), static_cast<void *>(b->d_items),
-                    static_cast<void *>(b->d_counter), static_cast<void *>(b->d_partials)})
+                    static_cast<void *>(b->d_counter), static_cast<void *>(b->d_partials),
+                    static_cast<void *>(b->d_columns), static_cast<void *>(b->d_slab)})
         if (p)
             (void)hipFree(p);
     b->d_ops = nullptr;
     b->d_items = nullptr;
     b->d_counter = nullptr;
     b->d_partials = nullptr;
-    b->cap_ops = b->cap_items = b->cap_partials = b->cap_counter = 0;
+    b->d_columns = b->d_slab = nullptr;
+    b->cap_ops = b->cap_items = b->cap_partials = b->cap_counter = b->cap_columns = b->cap_slab = 0;
 }
 
 template <class T> fp_status ensure_capacity(T **ptr, size_t &cap, size_t need, hipStream_t stream)
@@ -189,6 +202,12 @@ fp_status enqueue_kernels(fp_hip_batch *b, hipStream_t stream)
         if (r != FP_OK)
             return r;
     }
+    for (fprt::ColumnRound const &c : b->rounds)
+    {
+        fp_status const r = fprt::launch_column_round(c, b->d_columns, b->d_slab, b->d_slab + b->slab_bytes, stream);
+        if (r != FP_OK)
+            return r;
+    }
     return FP_OK;
 }
 
@@ -245,9 +264,55 @@ fp_status coset_plan(BatchEntry const &e, uint32_t min_kib, fprt::TileGeom *geo,
     return FP_OK;
 }
 
+// Columns of a round: as many bytes of outputs again.  Both are in the Infinity Cache (256 MB)
+// when the next kernel of the round reads them (256 entries, 3 GB: 32 MiB 19.9 ms, 64 MiB 19.1,
+// 128 MiB 18.9, 256 MiB 19.2, 512 MiB 19.4).
+constexpr size_t kRoundBytes = size_t(128) << 20;
+
+// Entries of at least this many bytes of states and terms (strings x elements) run on columns
+// whatever the schedule's thresholds; smaller ones where those leave them to the streaming items
+// and all the candidates of the batch are worth the launches of their rounds, three for each
+// variant (streaming items: about 1 ms for 1e9 terms).
+constexpr size_t kColumnsFirstBytes = size_t(4) << 20;
+constexpr double kColumnsFirstTerms = 3e7, kColumnsAllTerms = 5e8;
+
+double entry_terms(BatchEntry const &e)
+{
+    return double(e.ops->n_strings) * double(e.dim) * double(e.n_states);
+}
+
+// Tables and slabs of the entries on columns; FP_ERR_OUT_OF_MEMORY: no room for them.
+fp_status build_columns(fp_hip_batch *b, std::vector<fprt::ColumnEntry> const &entries, hipStream_t stream)
+{
+    b->rounds.clear();
+    b->column_entries = entries.size();
+    if (entries.empty())
+        return FP_OK;
+    size_t used = 0;
+    fprt::build_column_rounds(entries, kRoundBytes, b->rounds, b->h_columns, used);
+    fp_status const st = ensure_capacity(&b->d_columns, b->cap_columns, b->h_columns.size(), stream);
+    if (st != FP_OK)
+        return st;
+    if (b->cap_slab < 2 * used)
+    {
+        if (b->d_slab)
+        {
+            FP_HIP(hipStreamSynchronize(stream));
+            FP_HIP(hipFree(b->d_slab));
+        }
+        b->d_slab = nullptr;
+        b->cap_slab = 0;
+        FP_HIP(hipMalloc(reinterpret_cast<void **>(&b->d_slab), 2 * used));
+        b->cap_slab = 2 * used;
+    }
+    b->slab_bytes = used;
+    FP_HIP(hipMemcpyAsync(b->d_columns, b->h_columns.data(), b->h_columns.size(), hipMemcpyHostToDevice, stream));
+    return FP_OK;
+}
+
 // Cuts the entries into tiles, uploads the tables on `stream` and (in graph
 // mode) captures the launch.  The previous launch must have completed.
-fp_status build(fp_hip_batch *b, hipStream_t stream)
+fp_status build(fp_hip_batch *b, hipStream_t stream, bool columns)
 {
     wait_idle(b);
     drop_graph(b);
@@ -271,10 +336,19 @@ fp_status build(fp_hip_batch *b, hipStream_t stream)
         double bytes;
     };
     std::vector<CosetOp> coset_ops;
+    std::vector<fprt::ColumnEntry> column_entries;
     uint64_t partial_elems = 0;
     uint32_t n_deps = 0;
     bool any_expect = false;
     fp_hip_batch_schedule const &sc = b->sched;
+    auto column_candidate = [&](BatchEntry const &e) {
+        return columns && e.kind == FP_BATCH_APPLY && e.dim == (size_t(1) << e.ops->n_qubits) &&
+               fprt::batch_columns_eligible(e.ops, e.dtype, e.n_states);
+    };
+    double column_terms = 0.0;
+    for (BatchEntry const &e : b->entries)
+        if (column_candidate(e))
+            column_terms += entry_terms(e);
     for (size_t i = 0; i < b->entries.size(); ++i)
     {
         BatchEntry &e = b->entries[i];
@@ -307,6 +381,23 @@ fp_status build(fp_hip_batch *b, hipStream_t stream)
         op.accumulate = e.accumulate ? 1u : 0u;
         fprt::TileGeom geo{};
         fprt::TileTables *tt = nullptr;
+        bool const column_shape = column_candidate(e);
+        auto to_columns = [&] {
+            column_entries.push_back(fprt::ColumnEntry{
+                uint32_t(o->n_qubits), uint32_t(o->n_strings), e.dtype != FP_C128, e.accumulate != 0, e.n_states,
+                reinterpret_cast<uintptr_t>(e.states), reinterpret_cast<uintptr_t>(e.out),
+                reinterpret_cast<uintptr_t>(o->d_xz), reinterpret_cast<uintptr_t>(op.cf)});
+            // inputs read, columns written and read, outputs likewise (read first when accumulating)
+            b->plan_bytes += double(entry_in_bytes(e)) * (e.accumulate ? 9.0 : 6.0);
+            op.sshift = 64u;
+            op.n_tiles = 0;
+            ops.push_back(op);
+        };
+        if (column_shape && entry_in_bytes(e) >= kColumnsFirstBytes && entry_terms(e) >= kColumnsFirstTerms)
+        {
+            to_columns();
+            continue;
+        }
         if (e.kind == FP_BATCH_APPLY && sc.tiled_min_kib != 0)
         {
             fp_status ts = fprt::apply_tiled_plan(o, e.dtype, e.n_states, size_t(sc.tiled_min_kib) << 10,
@@ -368,6 +459,11 @@ fp_status build(fp_hip_batch *b, hipStream_t stream)
             b->coset_groups += tt->n_groups;
             ++b->coset_entries;
             ops.push_back(op);
+            continue;
+        }
+        if (column_shape && column_terms >= kColumnsAllTerms)
+        {
+            to_columns();
             continue;
         }
         op.ct = uint32_t(std::min<uint64_t>(g.vpr, fpk::kBlock));
@@ -510,7 +606,14 @@ fp_status build(fp_hip_batch *b, hipStream_t stream)
         b->n_blocks = uint32_t(std::max<int>(1, device_cus() * per_cu));
     }
 
-    fp_status st;
+    fp_status st = build_columns(b, column_entries, stream);
+    if (st == FP_ERR_OUT_OF_MEMORY && columns)
+    {
+        (void)hipGetLastError();
+        return build(b, stream, false);
+    }
+    if (st != FP_OK)
+        return st;
     if ((st = ensure_capacity(&b->d_ops, b->cap_ops, ops.size(), stream)) != FP_OK ||
         (st = ensure_capacity(&b->d_items, b->cap_items, std::max<size_t>(work.size(), 1), stream)) != FP_OK ||
         (st = ensure_capacity(&b->d_partials, b->cap_partials, std::max<uint64_t>(partial_elems, 1), stream)) !=
@@ -527,7 +630,8 @@ fp_status build(fp_hip_batch *b, hipStream_t stream)
                               hipMemcpyHostToDevice, stream));
     if (b->use_graph)
     {
-        // capture [reset, persistent kernel] once; replayed by every launch
+        // capture [reset, persistent kernel, launches of single entries, rounds of columns]
+        // once; replayed by every launch
         if (!b->capture_stream)
             FP_HIP(hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking));
         FP_HIP(hipStreamSynchronize(stream)); // tables uploaded before the graph can run on any stream
@@ -554,6 +658,13 @@ fp_status build(fp_hip_batch *b, hipStream_t stream)
 }
 
 } // namespace
+
+void fprt::batch_without_columns(fp_hip_batch *b)
+{
+    wait_idle(b);
+    drop_graph(b);
+    b->use_columns = false;
+}
 
 extern "C"
 {
@@ -707,6 +818,17 @@ fp_status fp_hip_batch_tiled_info(fp_hip_batch const *b, size_t *n_entries, size
     return FP_OK;
 }
 
+fp_status fp_hip_batch_column_info(fp_hip_batch const *b, size_t *n_entries, size_t *n_rounds)
+{
+    if (!b)
+        return fail(FP_ERR_INVALID_ARGUMENT, "batch is NULL");
+    if (n_entries)
+        *n_entries = b->column_entries;
+    if (n_rounds)
+        *n_rounds = b->rounds.size();
+    return FP_OK;
+}
+
 fp_status fp_hip_batch_check(fp_hip_batch *b)
 {
     if (!b)
@@ -736,10 +858,14 @@ fp_status fp_hip_batch_launch(fp_hip_batch *b, void *stream)
         }
     if (!b->built)
     {
-        fp_status const r = build(b, st);
+        fp_status const r = build(b, st, b->use_columns);
         if (r != FP_OK)
             return r;
     }
+    // launches on two streams would share the slabs
+    if (!b->rounds.empty() && b->last_done && b->last_stream != st)
+        FP_HIP(hipStreamWaitEvent(st, b->last_done, 0));
+    b->last_stream = st;
     if (b->use_graph)
         FP_HIP(hipGraphLaunch(b->exec, st));
     else

@@ -259,12 +259,17 @@ fp_status launch_apply_columns(void const *cols, void *out, uint32_t n, uint32_t
     return lds ? go(I8{}, I1{}, I1024{}, std::true_type{}) : go(I1{}, I4{}, I256{}, std::false_type{});
 }
 
-// The LDS tiles: columns of 2^9 to 2^14 rows, most of whose partner rows they hold, when the
-// tiles fill the chip; and columns as large as an XCD's L2 (2^18 rows of 16 bytes).
+// The LDS tiles (one block per CU): columns of 2^9 to 2^14 rows, at least half of whose partner
+// rows they hold, when whole rounds of them fill the chip.  us, LDS / direct: complex128, 500
+// strings, 1000 states n = 14 3180 / 4310, n = 12 716 / 1061, n = 14 300 states (600 tiles) 1131 /
+// 1300; but complex64 n = 14, 300 states (300 tiles) 816 / 670, and beyond, complex128 n = 18,
+// 30 states 2880 / 2520 (13 states 1575 / 1180, complex64 1630 / 846).
 bool apply_lds_tiles(uint32_t n, uint64_t n_cols)
 {
     uint64_t const tiles = n > 13 ? n_cols << (n - 13) : n_cols >> (13 - n);
-    return n >= 9 && (n <= 14 || n == 18) && tiles >= 192 && lds_bytes() >= (size_t(1) << 17);
+    uint64_t const rounds = (tiles + 255) / 256;
+    return n >= 9 && n <= 14 && tiles >= 192 && 10 * tiles >= 7 * 256 * rounds &&
+           lds_bytes() >= (size_t(1) << 17);
 }
 
 } // namespace
@@ -412,6 +417,60 @@ fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void con
         s = run(float{}, weighted ? ops->d_h64 : kind == kTilesSummedApply ? ops->d_rowsum64 : ops->d_cf64);
     *done = s == FP_OK;
     return s;
+}
+
+// Entries of a batch: columns as in apply_columns_route, but from 16 strings and 64 KiB of states,
+// as the copies and launches are shared.  256 complex64 entries, n = 8..18, 16..512 strings, 1..64
+// states, ms: from 32 strings and 4 MiB 26.2, 16 strings and 4 MiB 25.5, 1 MiB 24.2, 256 KiB 23.5,
+// 64 KiB 23.25, 16 KiB 23.2; 8 strings and 64 KiB 23.2.
+bool batch_columns_eligible(fp_hip_ops const *ops, int dtype, size_t n_states)
+{
+    size_t const n = ops->n_qubits, esz = dtype == FP_C128 ? 16 : 8;
+    char const *v = std::getenv("FAST_PAULI_APPLY_KERNEL");
+    if ((v && *v && std::strcmp(v, "columns") != 0) || n < 6 || n > 20 || n_states > (size_t(1) << 24))
+        return false;
+    size_t const col_bytes = (size_t(1) << n) * esz;
+    bool const pow2 = (n_states & (n_states - 1)) == 0;
+    return ops->n_strings >= 16 && col_bytes * n_states >= (size_t(64) << 10) &&
+           col_bytes <= (pow2 ? size_t(4) << 20 : size_t(8) << 20);
+}
+
+namespace
+{
+
+// f(type, states a row) for a variant of columns
+template <class F> fp_status with_columns(uint32_t variant, F f)
+{
+    if (!(variant & kColsC64))
+        return f(double{}, std::integral_constant<int, 1>{});
+    if (variant & kColsPairs)
+        return f(float{}, std::integral_constant<int, 2>{});
+    return f(float{}, std::integral_constant<int, 1>{});
+}
+
+} // namespace
+
+fp_status launch_column_round(ColumnRound const &r, unsigned char const *tables, unsigned char *in,
+                              unsigned char *out, hipStream_t st)
+{
+    auto const *jobs = reinterpret_cast<fpc::ColJob const *>(tables + r.o_jobs);
+    auto const *ends = reinterpret_cast<uint32_t const *>(tables + r.o_ends);
+    auto const *segs = reinterpret_cast<fpc::ColSeg const *>(tables + r.o_segs);
+    auto copies = [&](size_t o) { return reinterpret_cast<fpc::ColCopy const *>(tables + o); };
+    auto copy_ends = [&](size_t o) { return reinterpret_cast<uint32_t const *>(tables + o); };
+    return with_columns(r.variant, [&](auto T_tag, auto ns_tag) -> fp_status {
+        typedef decltype(T_tag) T;
+        constexpr int NS = decltype(ns_tag)::value;
+        hipLaunchKernelGGL((fpc::k_columns_batch<T, NS, true>), dim3(r.in_blocks), dim3(256), 0, st, in, out,
+                           copies(r.o_in), copy_ends(r.o_in_ends), r.n_in);
+        FP_LAUNCHED();
+        hipLaunchKernelGGL((fpc::k_apply_columns_batch<T, NS>), dim3(r.blocks), dim3(256), 0, st, in, out, jobs, ends, segs, r.n_segs);
+        FP_LAUNCHED();
+        hipLaunchKernelGGL((fpc::k_columns_batch<T, NS, false>), dim3(r.out_blocks), dim3(256), 0, st, in, out,
+                           copies(r.o_out), copy_ends(r.o_out_ends), r.n_out);
+        FP_LAUNCHED();
+        return FP_OK;
+    });
 }
 
 } // namespace fprt

@@ -352,25 +352,25 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
 }
 
 // Columns [c0, c0 + n_cols) of a row-major (rows x ld) batch to columns of NS states a row, and
-// back (IN = false).  Tiles of 32 rows x 32 states through LDS; an odd last state is paired with
-// zeros, which are not written back.
+// back (IN = false): block (bx, by) moves 32 rows of 32 states through LDS; an odd last state is
+// paired with zeros, which are not written back.
 template <class T, int NS, bool IN>
-__global__ __launch_bounds__(256) void k_columns(typename fpk::VecOf<T, 1>::type *__restrict__ batch,
-                                                 typename fpk::VecOf<T, NS>::type *__restrict__ cols, uint64_t rows,
-                                                 uint64_t ld, uint64_t c0, uint32_t n_cols)
+__device__ __forceinline__ void move_columns(__attribute__((address_space(1))) typename fpk::VecOf<T, 1>::type *batch,
+                                             typename fpk::VecOf<T, NS>::type *__restrict__ cols, uint64_t rows,
+                                             uint64_t ld, uint64_t c0, uint32_t n_cols, uint32_t bx, uint32_t by)
 {
     typedef typename fpk::VecOf<T, 1>::type V1;
     typedef typename fpk::VecOf<T, NS>::type V;
     __shared__ V1 tile[32][33];
-    uint64_t const r0 = uint64_t(blockIdx.x) * 32;
-    uint32_t const cb = blockIdx.y * 32u;
+    uint64_t const r0 = uint64_t(bx) * 32;
+    uint32_t const cb = by * 32u;
     uint32_t const tx = threadIdx.x & 31u, ty = threadIdx.x >> 5;
     auto batch_side = [&] {
 #pragma unroll
         for (uint32_t k = ty; k < 32; k += 8)
             if (r0 + k < rows)
             {
-                V1 *at = batch + (r0 + k) * ld + c0 + cb + tx;
+                auto *at = batch + (r0 + k) * ld + c0 + cb + tx;
                 bool const live = cb + tx < n_cols;
                 if constexpr (IN)
                     tile[k][tx] = live ? *at : V1(0);
@@ -413,6 +413,16 @@ __global__ __launch_bounds__(256) void k_columns(typename fpk::VecOf<T, 1>::type
         column_side();
     else
         batch_side();
+}
+
+template <class T, int NS, bool IN>
+__global__ __launch_bounds__(256) void k_columns(typename fpk::VecOf<T, 1>::type *__restrict__ batch,
+                                                 typename fpk::VecOf<T, NS>::type *__restrict__ cols, uint64_t rows,
+                                                 uint64_t ld, uint64_t c0, uint32_t n_cols)
+{
+    typedef typename fpk::VecOf<T, 1>::type V1;
+    move_columns<T, NS, IN>((__attribute__((address_space(1))) V1 *)batch, cols, rows, ld, c0, n_cols, blockIdx.x,
+                            blockIdx.y);
 }
 
 } // namespace fpc

@@ -200,6 +200,15 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
 int apply_columns_route(fp_hip_ops const *ops, int dtype, size_t n_states, bool weighted);
 fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void const *states, void const *data,
                             void *out, size_t dim, size_t n_states, int accumulate, hipStream_t st, bool *done);
+// The applies of a batch on columns, in rounds of one slab: whether an entry may take them, and
+// the launches of one round on tables and slabs in device memory (enqueues nothing else, so a
+// graph capture may record it).
+bool batch_columns_eligible(fp_hip_ops const *ops, int dtype, size_t n_states);
+fp_status launch_column_round(ColumnRound const &r, unsigned char const *tables, unsigned char *in,
+                              unsigned char *out, hipStream_t st);
+// Keeps the batch's applies off columns, whose slabs it would hold (a server's budget counts only
+// its requests' buffers).
+void batch_without_columns(fp_hip_batch *b);
 // Shape checks shared by the entry points.
 fp_status check_shape(fp_hip_ops const *ops, int dtype, void const *a, void const *b, size_t dim, size_t n_states);
 // Sets up the allocation-free entry point's static buffer on the current device

@@ -488,6 +488,8 @@ fp_status fp_hip_server_create(fp_hip_server **out, fp_serve_config const *cfg)
         fp_status st = fp_hip_batch_create(&sl.batch);
         if (st == FP_OK)
             st = fp_hip_batch_set_graph(sl.batch, 0);
+        if (st == FP_OK)
+            fprt::batch_without_columns(sl.batch);
         if (st != FP_OK)
             return st;
     }

@@ -240,5 +240,28 @@ struct XZ
     uint32_t x, z;
 };
 
+// Many operators on the columns of one slab (k_apply_columns_batch, k_columns_batch).
+struct ColJob
+{
+    uint64_t cols;   // byte offset of the first column in both slabs
+    uint64_t xz, cf; // device addresses of the operator's XZ records and folded coefficients
+    uint32_t n, n_cols, n_strings, accumulate;
+};
+// Blocks [block0, ...) of a job, from position `start` of an XCD's queue on.
+struct ColSeg
+{
+    uint32_t start, job, block0, pad;
+};
+// States [c0, c0 + n_states) of a row-major (2^n x ld) batch and their columns.
+struct ColCopy
+{
+    uint64_t batch; // device address
+    uint64_t cols;  // byte offset of the first column in its slab
+    uint64_t ld, c0;
+    uint32_t n, n_states;
+    uint32_t start; // first block
+    uint32_t out;   // the output slab's columns
+};
+
 } // namespace fpc
 

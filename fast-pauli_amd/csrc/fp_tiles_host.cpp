@@ -694,4 +694,164 @@ fp_status build_column_image(StringTable const &st, bool c64, uint32_t per_item,
     return FP_OK;
 }
 
+namespace
+{
+
+// Appends `count` records at a 256-byte boundary of the image.
+template <class R> size_t append(std::vector<unsigned char> &image, R const *r, size_t count)
+{
+    size_t const at = (image.size() + 255) / 256 * 256;
+    image.resize(at + count * sizeof(R));
+    if (count)
+        std::memcpy(image.data() + at, r, count * sizeof(R));
+    return at;
+}
+
+// Block ends padded with the last one to a multiple of 64 (and at least 64).
+void pad_ends(std::vector<uint32_t> &ends, size_t to)
+{
+    ends.resize(to, ends.empty() ? 0u : ends.back());
+}
+
+size_t round64(size_t v)
+{
+    return std::max<size_t>((v + 63) / 64 * 64, 64);
+}
+
+} // namespace
+
+void build_column_rounds(std::vector<ColumnEntry> const &entries, size_t slab_bytes,
+                         std::vector<ColumnRound> &rounds, std::vector<unsigned char> &image, size_t &used)
+{
+    rounds.clear();
+    image.clear();
+    used = 0;
+    // complex64 takes two states a row while such a column fits an XCD's L2
+    auto variant_of = [](ColumnEntry const &e) -> uint32_t {
+        return !e.c64 ? 0u : e.n <= 18 ? uint32_t(kColsC64 | kColsPairs) : uint32_t(kColsC64);
+    };
+    auto columns = [&](ColumnEntry const &e) -> uint64_t {
+        return (variant_of(e) & kColsPairs) ? (e.n_states + 1) / 2 : e.n_states;
+    };
+    std::vector<uint32_t> variant(entries.size());
+    std::vector<size_t> order(entries.size());
+    for (size_t i = 0; i < entries.size(); ++i)
+    {
+        variant[i] = variant_of(entries[i]);
+        order[i] = i;
+    }
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) {
+        return variant[a] != variant[b] ? variant[a] > variant[b] : entries[a].n_strings > entries[b].n_strings;
+    });
+
+    size_t k = 0;
+    uint64_t done = 0; // columns of entry order[k] in earlier rounds
+    while (k < order.size())
+    {
+        ColumnRound r{};
+        r.variant = variant[order[k]];
+        bool const pairs = (r.variant & kColsPairs) != 0;
+        uint32_t const tile = 8; // log2 rows of a block
+        uint64_t const row_bytes = !(r.variant & kColsC64) || pairs ? 16 : 8;
+        std::vector<fpc::ColJob> jobs;
+        std::vector<uint64_t> job_blocks;
+        std::vector<fpc::ColCopy> in, out;
+        std::vector<uint32_t> in_ends, out_ends;
+        uint64_t at = 0;
+        double cost = 0.0;
+        while (k < order.size() && variant[order[k]] == r.variant)
+        {
+            ColumnEntry const &e = entries[order[k]];
+            uint64_t const col_bytes = row_bytes << e.n, all = columns(e);
+            uint64_t const room = at < slab_bytes ? (slab_bytes - at) / col_bytes : 0;
+            uint64_t const take = std::min<uint64_t>(all - done, std::max<uint64_t>(room, at == 0 ? 1 : 0));
+            if (take == 0)
+                break;
+            uint64_t const c0 = pairs ? 2 * done : done;
+            uint64_t const ns = std::min<uint64_t>(pairs ? 2 * take : take, e.n_states - c0);
+            jobs.push_back(fpc::ColJob{at, e.xz, e.cf, e.n, uint32_t(take), e.n_strings, e.accumulate ? 1u : 0u});
+            // blocks: the tiles of each column, or the groups of columns that fill a tile
+            job_blocks.push_back(e.n > tile ? take << (e.n - tile)
+                                            : (take + (uint64_t(1) << (tile - e.n)) - 1) >> (tile - e.n));
+            cost += double(job_blocks.back()) * e.n_strings;
+            uint32_t const copy_blocks = uint32_t(((uint64_t(1) << e.n) + 31) / 32 * ((ns + 31) / 32));
+            fpc::ColCopy const c{0, at, e.n_states, c0, e.n, uint32_t(ns), 0, 0};
+            auto add = [&](std::vector<fpc::ColCopy> &list, std::vector<uint32_t> &ends, uint32_t &blocks,
+                           uint64_t batch, uint32_t to_out) {
+                list.push_back(c);
+                list.back().batch = batch;
+                list.back().start = blocks;
+                list.back().out = to_out;
+                blocks += copy_blocks;
+                ends.push_back(blocks);
+            };
+            add(in, in_ends, r.in_blocks, e.states, 0);
+            if (e.accumulate)
+                add(in, in_ends, r.in_blocks, e.out, 1);
+            add(out, out_ends, r.out_blocks, e.out, 1);
+            at += (take * col_bytes + 255) / 256 * 256;
+            done += take;
+            if (done < all)
+                break; // the slab is full
+            done = 0;
+            ++k;
+        }
+        used = std::max<size_t>(used, at);
+        // every XCD's queue: an eighth of the round's string terms, cut between blocks
+        std::vector<std::vector<fpc::ColSeg>> segs(8);
+        std::vector<std::vector<uint32_t>> ends(8);
+        size_t j = 0;
+        uint64_t b = 0; // next block of job j
+        double taken = 0.0;
+        for (uint32_t x = 0; x < 8; ++x)
+        {
+            double const goal = cost * double(x + 1) / 8.0;
+            uint32_t pos = 0;
+            while (j < jobs.size() && (x == 7 || taken < goal))
+            {
+                double const per = jobs[j].n_strings;
+                uint64_t n = job_blocks[j] - b;
+                if (x < 7)
+                    n = std::min<uint64_t>(n, std::max<uint64_t>(1, uint64_t((goal - taken) / per + 0.5)));
+                segs[x].push_back(fpc::ColSeg{pos, uint32_t(j), uint32_t(b), 0});
+                pos += uint32_t(n);
+                ends[x].push_back(pos);
+                taken += double(n) * per;
+                b += n;
+                if (b == job_blocks[j])
+                {
+                    ++j;
+                    b = 0;
+                }
+            }
+            r.blocks = std::max(r.blocks, 8 * pos);
+        }
+        size_t most = 0;
+        for (auto const &s : segs)
+            most = std::max(most, s.size());
+        r.n_segs = uint32_t(round64(most));
+        std::vector<uint32_t> all_ends;
+        std::vector<fpc::ColSeg> all_segs;
+        for (uint32_t x = 0; x < 8; ++x)
+        {
+            pad_ends(ends[x], r.n_segs);
+            segs[x].resize(r.n_segs);
+            all_ends.insert(all_ends.end(), ends[x].begin(), ends[x].end());
+            all_segs.insert(all_segs.end(), segs[x].begin(), segs[x].end());
+        }
+        r.n_in = uint32_t(in.size());
+        r.n_out = uint32_t(out.size());
+        pad_ends(in_ends, round64(in_ends.size()));
+        pad_ends(out_ends, round64(out_ends.size()));
+        r.o_jobs = append(image, jobs.data(), jobs.size());
+        r.o_ends = append(image, all_ends.data(), all_ends.size());
+        r.o_segs = append(image, all_segs.data(), all_segs.size());
+        r.o_in = append(image, in.data(), in.size());
+        r.o_in_ends = append(image, in_ends.data(), in_ends.size());
+        r.o_out = append(image, out.data(), out.size());
+        r.o_out_ends = append(image, out_ends.data(), out_ends.size());
+        rounds.push_back(r);
+    }
+}
+
 } // namespace fprt

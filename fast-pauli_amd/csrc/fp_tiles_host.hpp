@@ -83,4 +83,35 @@ fp_status build_tile_image(StringTable const &st, int kind, uint32_t k, uint32_t
 // string evaluations of a whole tile (n_groups items).
 fp_status build_column_image(StringTable const &st, bool c64, uint32_t per_item, TileImage &out);
 
+// An apply of a batch that runs on columns.  Addresses are device addresses: the states and
+// outputs, and the operator's fpc::XZ records and folded coefficients of its type.
+struct ColumnEntry
+{
+    uint32_t n, n_strings;
+    bool c64, accumulate;
+    uint64_t n_states;
+    uint64_t states, out, xz, cf;
+};
+
+// The launches of one slab of columns: copies in, one apply kernel, copies out.
+enum
+{
+    kColsC64 = 1,  // complex64
+    kColsPairs = 2 // two states a row
+};
+struct ColumnRound
+{
+    uint32_t variant; // kCols* bits
+    uint32_t blocks, n_segs;
+    uint32_t n_in, in_blocks, n_out, out_blocks;
+    // offsets into the image: fpc::ColJob, uint32_t ends, fpc::ColSeg (n_segs per XCD), and
+    // fpc::ColCopy with their uint32_t ends
+    size_t o_jobs, o_ends, o_segs, o_in, o_in_ends, o_out, o_out_ends;
+};
+
+// Cuts the entries into rounds of at most `slab_bytes` of columns of one variant, longest
+// operators first, so that the blocks of a round last about as long.  `used`: the bytes of columns of the largest round.
+void build_column_rounds(std::vector<ColumnEntry> const &entries, size_t slab_bytes,
+                         std::vector<ColumnRound> &rounds, std::vector<unsigned char> &image, size_t &used);
+
 } // namespace fprt

@@ -183,6 +183,7 @@ _SIGS.update({
     "fp_hip_batch_coset_info": [_vp, ctypes.POINTER(_sz), ctypes.POINTER(_sz), ctypes.POINTER(_sz),
                                 ctypes.POINTER(ctypes.c_double)],
     "fp_hip_batch_tiled_info": [_vp, ctypes.POINTER(_sz), ctypes.POINTER(_sz)],
+    "fp_hip_batch_column_info": [_vp, ctypes.POINTER(_sz), ctypes.POINTER(_sz)],
     "fp_hip_batch_check": [_vp],
     "fp_hip_batch_launch": [_vp, _vp],
     "fp_hip_batch_set_graph": [_vp, _i],

@@ -82,9 +82,12 @@ class Batch:
                   ctypes.byref(pb))
         te, tg = ctypes.c_size_t(), ctypes.c_size_t()
         _abi.call("fp_hip_batch_tiled_info", self.handle, ctypes.byref(te), ctypes.byref(tg))
+        ce, cr = ctypes.c_size_t(), ctypes.c_size_t()
+        _abi.call("fp_hip_batch_column_info", self.handle, ctypes.byref(ce), ctypes.byref(cr))
         return {"entries": a.value, "tiles": b.value, "blocks": c.value,
                 "coset_entries": e.value, "coset_groups": g.value, "coset_items": i.value,
-                "tiled_entries": te.value, "tiled_groups": tg.value, "plan_bytes": pb.value}
+                "tiled_entries": te.value, "tiled_groups": tg.value,
+                "column_entries": ce.value, "column_rounds": cr.value, "plan_bytes": pb.value}
 
     def check(self) -> None:
         """Waits for the last launch; raises if a coset item gave up waiting for its

@@ -170,6 +170,147 @@ cplx through_tables(Set const &s, bool c64, uint32_t per_item, std::vector<cplx>
     return sum;
 }
 
+// Rounds of a batch: through the tables, as the kernels walk them, every state of every entry is
+// copied in once (outputs too when accumulating), computed by exactly the blocks that cover its
+// column, and copied out once; columns of a round stay apart and inside the slab.
+int check_rounds(std::vector<fprt::ColumnEntry> const &es, size_t slab)
+{
+    std::vector<fprt::ColumnRound> rounds;
+    std::vector<unsigned char> im;
+    size_t used = 0;
+    fprt::build_column_rounds(es, slab, rounds, im, used);
+    int bad = 0;
+    std::vector<std::vector<int>> in(es.size()), acc(es.size()), out(es.size());
+    for (size_t i = 0; i < es.size(); ++i)
+        for (auto *v : {&in[i], &acc[i], &out[i]})
+            v->assign(es[i].n_states, 0);
+    auto find = [](uint32_t const *ends, uint32_t count, uint32_t pos) {
+        uint32_t i = 0;
+        while (i < count && pos >= ends[i])
+            ++i;
+        return i;
+    };
+    for (fprt::ColumnRound const &r : rounds)
+    {
+        auto const *jobs = reinterpret_cast<fpc::ColJob const *>(im.data() + r.o_jobs);
+        bool const pairs = r.variant & fprt::kColsPairs;
+        uint32_t const tile = 8;
+        uint64_t const row = (r.variant & fprt::kColsC64) && !pairs ? 8 : 16;
+        // copies: block by block
+        struct Span
+        {
+            uint64_t at, size;
+            size_t entry;
+        };
+        std::vector<Span> spans;
+        for (int dir = 0; dir < 2; ++dir)
+        {
+            auto const *c = reinterpret_cast<fpc::ColCopy const *>(im.data() + (dir ? r.o_out : r.o_in));
+            auto const *ends = reinterpret_cast<uint32_t const *>(im.data() + (dir ? r.o_out_ends : r.o_in_ends));
+            uint32_t const count = dir ? r.n_out : r.n_in, blocks = dir ? r.out_blocks : r.in_blocks;
+            std::vector<uint32_t> seen(count, 0);
+            for (uint32_t b = 0; b < blocks; ++b)
+            {
+                uint32_t const at = find(ends, count, b);
+                if (at >= count)
+                {
+                    ++bad;
+                    continue;
+                }
+                bad += b - c[at].start != seen[at]++;
+            }
+            for (uint32_t k = 0; k < count; ++k)
+            {
+                fpc::ColCopy const &k_ = c[k];
+                size_t e = 0;
+                while (e < es.size() && (k_.out ? es[e].out : es[e].states) != k_.batch)
+                    ++e;
+                if (e == es.size())
+                {
+                    ++bad;
+                    continue;
+                }
+                bad += k_.n != es[e].n || k_.ld != es[e].n_states;
+                bad += seen[k] != ((uint64_t(1) << k_.n) + 31) / 32 * ((k_.n_states + 31) / 32);
+                auto &v = dir ? out[e] : k_.out ? acc[e] : in[e];
+                for (uint64_t t = 0; t < k_.n_states; ++t)
+                    ++v.at(k_.c0 + t);
+                uint64_t const cols = pairs ? (k_.n_states + 1) / 2 : k_.n_states;
+                bad += pairs && k_.c0 % 2 != 0;
+                bad += k_.cols + cols * (row << k_.n) > used || k_.cols % 16 != 0;
+                if (dir)
+                    spans.push_back(Span{k_.cols, cols * (row << k_.n), e});
+            }
+        }
+        for (size_t a = 0; a < spans.size(); ++a)
+            for (size_t b = 0; b < a; ++b)
+                bad += spans[a].at < spans[b].at + spans[b].size && spans[b].at < spans[a].at + spans[a].size;
+        // apply blocks
+        auto const *ends = reinterpret_cast<uint32_t const *>(im.data() + r.o_ends);
+        auto const *segs = reinterpret_cast<fpc::ColSeg const *>(im.data() + r.o_segs);
+        bad += r.n_segs % 64 != 0 || r.blocks % 8 != 0;
+        std::vector<std::vector<int>> hit(spans.size());
+        for (size_t j = 0; j < spans.size(); ++j)
+        {
+            fprt::ColumnEntry const &e = es[spans[j].entry];
+            bad += jobs[j].cols != spans[j].at || jobs[j].n != e.n || jobs[j].n_strings != e.n_strings ||
+                   jobs[j].xz != e.xz || jobs[j].cf != e.cf || (jobs[j].accumulate != 0) != e.accumulate ||
+                   jobs[j].n_cols * (row << e.n) != spans[j].size;
+            uint64_t const per = e.n < tile ? 1u << (tile - e.n) : 1u, tiles = e.n > tile ? 1u << (e.n - tile) : 1u;
+            hit[j].assign((jobs[j].n_cols + per - 1) / per * tiles, 0);
+        }
+        for (uint32_t b = 0; b < r.blocks; ++b)
+        {
+            uint32_t const x = b & 7, pos = b >> 3, at = find(ends + x * r.n_segs, r.n_segs, pos);
+            if (at >= r.n_segs)
+                continue;
+            fpc::ColSeg const &s = segs[x * r.n_segs + at];
+            ++hit.at(s.job).at(s.block0 + pos - s.start);
+        }
+        for (auto const &h : hit)
+            for (int v : h)
+                bad += v != 1;
+    }
+    for (size_t i = 0; i < es.size(); ++i)
+        for (size_t t = 0; t < es[i].n_states; ++t)
+            bad += in[i][t] != 1 || out[i][t] != 1 || acc[i][t] != (es[i].accumulate ? 1 : 0);
+    bad += used > slab && es.size() > 1; // (a lone column may be larger than the slab)
+    return bad;
+}
+
+int round_cases(Rng &r)
+{
+    int n_cases = 0;
+    for (size_t slab : {size_t(1) << 14, size_t(1) << 18, size_t(1) << 22})
+        for (int rep = 0; rep < 2; ++rep)
+            for (size_t count : {size_t(1), size_t(2), size_t(9), size_t(150)})
+            {
+                std::vector<fprt::ColumnEntry> es;
+                for (size_t i = 0; i < count; ++i)
+                {
+                    fprt::ColumnEntry e{};
+                    e.n = 6 + uint32_t(r.next() % (slab >= (size_t(1) << 22) ? 13 : 5));
+                    e.n_strings = 1 + uint32_t(r.next() % 600);
+                    e.c64 = r.next() % 2;
+                    e.accumulate = r.next() % 3 == 0;
+                    e.n_states = 1 + r.next() % (count > 9 ? 9 : 70);
+                    e.states = 0x1000 * (4 * i + 1);
+                    e.out = 0x1000 * (4 * i + 2);
+                    e.xz = 0x1000 * (4 * i + 3);
+                    e.cf = 0x1000 * (4 * i + 4);
+                    es.push_back(e);
+                }
+                ++n_cases;
+                if (int const bad = check_rounds(es, slab))
+                {
+                    ++g_failures;
+                    std::fprintf(stderr, "FAIL rounds slab=%zu count=%zu: %d faults\n", slab, count,
+                                 bad);
+                }
+            }
+    return n_cases;
+}
+
 } // namespace
 
 int main()
@@ -197,6 +338,7 @@ int main()
                     }
                 }
         }
+    n_cases += round_cases(r);
     // sizes the kernel does not take
     Set const small = make(fpc::low_bits(false) - 1, 4, 0, r), large = make(fpc::tile_bits(false) + 13, 4, 0, r);
     fprt::TileImage im;

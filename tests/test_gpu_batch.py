@@ -334,3 +334,41 @@ def test_tiled_launch_entries_bit_exact(hip, graph):
         for e in big:
             assert np.array_equal(e.result(), e.alone())
     b.destroy()
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_column_entries_bit_exact(hip, graph):
+    """Apply entries run on columns, in rounds of one slab after the other entries: IEEE-equal to the operator alone, both types, one and two states a row (an odd
+    last state), LDS tiles and direct columns, more than one round, accumulating, beside
+    streaming and expectation entries, over replays; re-targeted sets are picked up."""
+    H.say(f"batch columns graph={graph}")
+    A, E = _abi.FP_BATCH_APPLY, _abi.FP_BATCH_EXPECT
+    specs = [
+        (A, 14, 64, 33, C64, False), (A, 18, 33, 3, C64, True), (A, 18, 32, 1, C128, False),
+        (A, 16, 40, 5, C128, True), (A, 12, 100, 129, C64, False), (A, 9, 64, 2100, C64, False),
+        (A, 6, 90, 9000, C64, False), (A, 11, 50, 200, C128, False), (A, 15, 37, 520, C64, False),
+        (A, 19, 32, 3, C64, False), (A, 14, 35, 16, C128, False), (A, 7, 48, 2100, C128, True),
+        (E, 10, 20, 7, C64, False), (A, 9, 12, 4, C64, False), (E, 12, 30, 16, C128, True),
+        (A, 16, 15, 9, C64, False),
+    ]
+    entries = [Entry(*s, seed=60 + i) for i, s in enumerate(specs)]
+    b = Batch()
+    if not graph:
+        _abi.call("fp_hip_batch_set_graph", b.handle, 0)
+    for e in entries:
+        b.add(e.kind, e.ops, e.d_in.ptr, e.d_out.ptr, 1 << e.n, e.S, e.dtype, e.accumulate)
+    for rep in range(3):
+        if rep == 2:  # new strings and coefficients in one set: the tables are rebuilt
+            e = entries[0]
+            codes, coeffs = syn.random_codes(70, e.n, seed=99), syn.random_coeffs(70, seed=99)
+            e.ops.assign(codes, coeffs)
+        for e in entries:
+            e.reset()
+        b.launch()
+        _abi.synchronize()
+        info = b.info()
+        assert info["column_entries"] == 12 and info["column_rounds"] == 4, info
+        assert info["tiles"] > 0, info
+        for e in entries:
+            check(e, e.result())
+    b.destroy()
