@@ -13,14 +13,19 @@
 // a per-lane offset (one XOR per string), a scalar offset per slot.  The sign is a per-lane bit,
 // a wave-uniform bit and one flip per slot, applied as the factor of the final multiply-add.
 //
-// Bound: about 10 vector instructions per (string, 64 rows), 8 of them the unfused product and
-// sums, against 16 clocks of L1 for a gathered KiB (64 bytes a clock; 4 clocks from LDS).  Two
-// shapes are built: one row a thread, partner rows gathered from L2 four strings ahead; and 2^13
-// rows a block in LDS (fp_columns.hip says which runs where).  Measured, row-major kernels /
-// columns, us: n = 10, 128 complex128 states, 64 strings 18.6 / 10.9; n = 18, one complex128
-// state, 1000 strings 287 / 144; n = 20, 19 complex64 states, 512 strings 10990 / 5780 (8 MiB a
-// column: past an XCD's L2); n = 14, 1000 complex128 states, 2000 strings, a weight per string
-// and state 29130 / 11520.
+// Bound: 12 to 14 vector instructions per (string, 64 rows), 8 of them the unfused product and
+// sums, against 16 clocks of L1 for a gathered KiB (64 bytes a clock; 4 clocks from LDS) and the
+// scalar unit, which all four SIMDs share: whole rounds of strings run without a branch, on
+// structure-of-arrays masks (wide scalar loads), and with one row a thread only a shift a string
+// is scalar.  Tests between the strings and masks split by scalar instructions made every wave
+// wait for its loads (n = 16, one complex128 state, 500 strings 40.6 us, now 19.3; n = 10, 128
+// states, 64 strings 8.5, now 6.9; n = 18, 13 complex64 states, 300 strings 524, now 397).  Two
+// shapes are built: one row a thread, partner rows gathered from L2 four or eight strings ahead;
+// and 2^13 rows a block in LDS (fp_columns.hip says which runs where).  Measured, row-major
+// kernels / columns, us: n = 10, 128 complex128 states, 64 strings 18.6 / 9.8; n = 18, one
+// complex128 state, 1000 strings 287 / 135; n = 20, 19 complex64 states, 512 strings 10990 / 5700
+// (8 MiB a column: past an XCD's L2); n = 14, 1000 complex128 states, 2000 strings, a weight per
+// string and state 29130 / 10800.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -90,13 +95,13 @@ template <class P> using Const = __attribute__((address_space(4))) P const;
 // (cols to out), NS states a row.  A block of TH threads owns a tile of TH * E rows of a column,
 // or the columns that fill it.
 // LDS: the tile's rows are kept in LDS, and strings whose partner rows lie in it read them there.
-// PIPE: the next strings' partner rows are in flight while U strings are added.
+// D: partner rows of D - 1 batches of U strings are in flight while one batch is added.
 // cf: complex coefficients with (-i)^{nY} folded in; WTD: those of state t at cf + 2 * cf_stride * t.
 // shift: masks are shifted by this many bits (one column made of a whole batch).
-template <class T, int NS, int E, int U, int TH, bool LDS, bool PIPE, bool WTD>
+template <class T, int NS, int E, int U, int TH, bool LDS, int D, bool WTD>
 __device__ __forceinline__ void apply_columns(BlockOf bo, typename fpk::VecOf<T, NS>::type const *__restrict__ cols,
                                               typename fpk::VecOf<T, NS>::type *__restrict__ out, uint32_t n,
-                                              uint32_t n_cols, Const<XZ> *xz, Const<T> *cf, uint64_t cf_stride,
+                                              uint32_t n_cols, Const<uint32_t> *xs, Const<uint32_t> *zs, Const<T> *cf, uint64_t cf_stride,
                                               uint32_t n_states, uint32_t n_strings, uint32_t shift, int accumulate)
 {
     typedef typename fpk::VecOf<T, NS>::type V; // one row of NS states
@@ -140,38 +145,44 @@ __device__ __forceinline__ void apply_columns(BlockOf bo, typename fpk::VecOf<T,
         c[w] = cf + 2 * cf_stride * (WTD ? (tc * NS + w < n_states ? tc * NS + w : n_states - 1u) : 0u);
     __amdgpu_buffer_rsrc_t const rsrc = column_rsrc(col, rows);
     uint32_t const lv = lane << kLv, gv = g << (kLow + kLv);
-    // Three stages: the records of batch k + 2 (scalar loads), the partner rows of batch
-    // k + 1, the terms of batch k.  Records past the end are read (the tables are padded)
-    // and their partner rows too (inside the column, or zero), but add nothing.
-    struct Rec
-    {
-        XZ q;
-        T cr[WTD ? NS : 1], ci[WTD ? NS : 1];
+    uint32_t const rv = row0 << kLv, rz = row0 >> shift; // one row a thread: its offset, its bits for z
+    // Batches of U strings in a pipeline: while batch k is added, the partner rows of the next
+    // D - 1 batches are in flight, and the scalar loads of x for batch k + D and of z and the
+    // coefficients for k + 1.  Masks and coefficients are read past the end (the tables are
+    // padded), and rows with them (inside the column, or zero), but add nothing.
+    constexpr int Q = D == 3 ? 3 : 2; // batches a round, and buffers of scalars
+    uint32_t x[Q][U], z[Q][U];
+    T cr[Q][U][WTD ? NS : 1], ci[Q][U][WTD ? NS : 1];
+    V R[D][U][E];
+    auto fetch_x = [&](int k, uint32_t(&v)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            v[u] = xs[k * U + u];
     };
-    Rec rec[3][U];
-    V R[PIPE ? 2 : 1][U][E];
-    Const<XZ> *qp = xz;
-    auto fetch = [&](int k, Rec(&r)[U]) {
+    auto fetch_c = [&](int k, uint32_t(&v)[U], T(&r)[U][WTD ? NS : 1], T(&i)[U][WTD ? NS : 1]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
         {
-            r[u].q = XZ{qp[k * U + u].x << shift, qp[k * U + u].z << shift};
+            v[u] = zs[k * U + u];
 #pragma unroll
             for (int w = 0; w < (WTD ? NS : 1); ++w)
             {
-                r[u].cr[w] = c[w][2 * (k * U + u)];
-                r[u].ci[w] = c[w][2 * (k * U + u) + 1];
+                r[u][w] = c[w][2 * (k * U + u)];
+                i[u][w] = c[w][2 * (k * U + u) + 1];
             }
         }
     };
-    auto load = [&](Rec const(&r)[U], V(&v)[U][E]) {
+    auto load = [&](uint32_t const(&xv)[U], V(&v)[U][E]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
         {
-            uint32_t const x = r[u].q.x;
-            if (LDS && (x >> kTile) == 0)
+            // one row a thread: its whole offset in a vector register (one scalar instruction a
+            // string; the lane and wave parts take several, which E rows share)
+            if constexpr (E == 1)
+                v[u][0] = buffer_load<V>(rsrc, rv ^ (xv[u] << (shift + kLv)), 0);
+            else if (uint32_t const xu = xv[u] << shift; LDS && (xu >> kTile) == 0)
             {
-                uint32_t const a = a0 ^ (x << kLv);
+                uint32_t const a = a0 ^ (xu << kLv);
 #pragma unroll
                 for (int i = 0; i < E; ++i)
                     v[u][i] =
@@ -179,25 +190,27 @@ __device__ __forceinline__ void apply_columns(BlockOf bo, typename fpk::VecOf<T,
             }
             else
             {
-                uint32_t const vo = lv ^ ((x & 63u) << kLv), so = gv ^ ((x >> 6) << (6u + kLv));
+                uint32_t const vo = lv ^ ((xu & 63u) << kLv), so = gv ^ ((xu >> 6) << (6u + kLv));
 #pragma unroll
                 for (int i = 0; i < E; ++i)
                     v[u][i] = buffer_load<V>(rsrc, vo, so ^ (uint32_t(i) * kSlot));
             }
         }
     };
-    auto eval = [&](uint32_t s0, Rec const(&r)[U], V(&v)[U][E]) {
+    auto eval = [&](uint32_t count, uint32_t const(&zv)[U], T const(&r)[U][WTD ? NS : 1],
+                    T const(&im)[U][WTD ? NS : 1], V(&v)[U][E]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (s0 + uint32_t(u) < n_strings)
+            if (uint32_t(u) < count)
             {
-                uint32_t const z = r[u].q.z;
                 // sign of the row: per-lane bits, wave-uniform bits, then one flip per slot
-                uint32_t const neg = uint32_t(__popc(lane & z)) + uint32_t(__popc(g & (z >> kLow)));
+                uint32_t const zu = zv[u] << shift;
+                uint32_t const neg = E == 1 ? uint32_t(__popc(rz & zv[u]))
+                                            : uint32_t(__popc(lane & zu)) + uint32_t(__popc(g & (zu >> kLow)));
                 uint32_t zb[kLe + 1];
 #pragma unroll
                 for (uint32_t b = 0; b < kLe; ++b)
-                    zb[b] = (z << (25u - b)) & 0x80000000u;
+                    zb[b] = (zu << (25u - b)) & 0x80000000u;
                 T sg = unit_sign<T>(neg << 31);
                 // slots in Gray-code order: one sign flip from each to the next
 #pragma unroll
@@ -213,41 +226,51 @@ __device__ __forceinline__ void apply_columns(BlockOf bo, typename fpk::VecOf<T,
                         // one rounding in the sum, which a multiply-add by +-1 gives exactly
                         int const w = WTD ? h : 0;
                         T tr, ti;
-                        fpk::cmul_exact<T>(r[u].cr[w], r[u].ci[w], v[u][i][2 * h], v[u][i][2 * h + 1], tr, ti);
+                        fpk::cmul_exact<T>(r[u][w], im[u][w], v[u][i][2 * h], v[u][i][2 * h + 1], tr, ti);
                         acc[i][2 * h] = fma(sg, tr, acc[i][2 * h]);
                         acc[i][2 * h + 1] = fma(sg, ti, acc[i][2 * h + 1]);
                     }
                 }
             }
     };
-    fetch(0, rec[0]);
-    fetch(1, rec[1]);
-    if constexpr (PIPE)
-        load(rec[0], R[0]);
-    for (uint32_t s0 = 0; s0 < n_strings; s0 += 6 * U)
+    auto step = [&](int k) {
+        fetch_c(k + 1, z[(k + 1) % Q], cr[(k + 1) % Q], ci[(k + 1) % Q]);
+        fetch_x(k + D, x[(k + D) % Q]);
+        load(x[(k + D - 1) % Q], R[(k + D - 1) % D]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int k = 0; k < D - 1; ++k)
+    {
+        fetch_x(k, x[0]);
+        load(x[0], R[k]);
+    }
+    fetch_x(D - 1, x[(D - 1) % Q]);
+    fetch_c(0, z[0], cr[0], ci[0]);
+    uint32_t left = n_strings;
+    for (; left >= uint32_t(Q * U); left -= Q * U) // whole rounds: no tests inside
     {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) // a multiple of both buffer counts
+        for (int k = 0; k < Q; ++k)
         {
-            uint32_t const sk = s0 + uint32_t(k) * U;
-            if (sk >= n_strings)
-                break;
-            fetch(k + 2, rec[(k + 2) % 3]);
-            if constexpr (PIPE)
-            {
-                if (sk + U < n_strings)
-                    load(rec[(k + 1) % 3], R[(k + 1) % 2]);
-            }
-            else
-                load(rec[k % 3], R[0]);
-            __builtin_amdgcn_sched_barrier(0);
-            eval(sk, rec[k % 3], R[PIPE ? k % 2 : 0]);
+            step(k);
+            eval(U, z[k % Q], cr[k % Q], ci[k % Q], R[k % D]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        qp += 6 * U;
+        xs += Q * U;
+        zs += Q * U;
 #pragma unroll
         for (int w = 0; w < (WTD ? NS : 1); ++w)
-            c[w] += 12 * U;
+            c[w] += 2 * Q * U;
+    }
+#pragma unroll
+    for (int k = 0; k < Q; ++k)
+    {
+        if (left <= uint32_t(k * U))
+            break;
+        step(k);
+        eval(left - uint32_t(k * U), z[k % Q], cr[k % Q], ci[k % Q], R[k % D]);
+        __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int i = 0; i < E; ++i)
@@ -256,16 +279,16 @@ __device__ __forceinline__ void apply_columns(BlockOf bo, typename fpk::VecOf<T,
 }
 
 // One operator on n_cols columns: n_groups * tiles blocks.
-template <class T, int NS, int E, int U, int TH, bool LDS, bool PIPE, bool WTD>
+template <class T, int NS, int E, int U, int TH, bool LDS, int D, bool WTD>
 __global__ __launch_bounds__(TH) void k_apply_columns(typename fpk::VecOf<T, NS>::type const *__restrict__ cols,
                                                       typename fpk::VecOf<T, NS>::type *__restrict__ out, uint32_t n,
                                                       uint32_t n_cols, uint32_t n_groups, uint32_t tiles,
-                                                      XZ const *__restrict__ xz, T const *__restrict__ cf,
+                                                      uint32_t const *__restrict__ xs, uint32_t const *__restrict__ zs, T const *__restrict__ cf,
                                                       uint64_t cf_stride, uint32_t n_states, uint32_t n_strings, uint32_t shift,
                                                       int accumulate)
 {
-    apply_columns<T, NS, E, U, TH, LDS, PIPE, WTD>(block_of(blockIdx.x, tiles, n_groups), cols, out, n, n_cols,
-                                                   (Const<XZ> *)xz, (Const<T> *)cf, cf_stride, n_states, n_strings,
+    apply_columns<T, NS, E, U, TH, LDS, D, WTD>(block_of(blockIdx.x, tiles, n_groups), cols, out, n, n_cols,
+                                                   (Const<uint32_t> *)xs, (Const<uint32_t> *)zs, (Const<T> *)cf, cf_stride, n_states, n_strings,
                                                    shift, accumulate);
 }
 
@@ -286,8 +309,9 @@ __device__ __forceinline__ uint32_t find_segment(uint32_t const *ends, uint32_t 
 // works through its own n_segs segments, so the blocks of a column follow each other on one XCD
 // and every XCD gets the same number of string terms, whatever the operators' sizes.  One row a
 // thread, straight from the columns: 256 complex64 operators of n = 8..18 (3 GB of states, 5.5e10
-// terms) take 18.9 ms, 57.3 as streaming items and coset-tiled launches, 23.2 with the LDS tiles
-// for n = 9..14 and 18 (19.2 for n = 9..14, whose blocks are too few to fill their rounds).
+// terms) take 18.0 ms, 57.3 as streaming items and coset-tiled launches; LDS tiles
+// made it 4.4 ms slower for n = 9..14 and 18 (0.3 ms for n = 9..14, whose blocks are too few to
+// fill their rounds).
 template <class T, int NS>
 __global__ __launch_bounds__(256) void k_apply_columns_batch(unsigned char const *__restrict__ in,
                                                              unsigned char *__restrict__ out,
@@ -305,9 +329,9 @@ __global__ __launch_bounds__(256) void k_apply_columns_batch(unsigned char const
     ColJob const j = jobs[sg.job];
     uint32_t const b = sg.block0 + (pos - sg.start);
     uint32_t const lt = j.n > kTile ? j.n - kTile : 0u; // log2 tiles of a column
-    apply_columns<T, NS, 1, 4, 256, false, true, false>(
+    apply_columns<T, NS, 1, 4, 256, false, 2, false>(
         BlockOf{b >> lt, b & ((1u << lt) - 1u)}, reinterpret_cast<V const *>(in + j.cols),
-        reinterpret_cast<V *>(out + j.cols), j.n, j.n_cols, (Const<XZ> *)j.xz, (Const<T> *)j.cf, 0, 0, j.n_strings, 0,
+        reinterpret_cast<V *>(out + j.cols), j.n, j.n_cols, (Const<uint32_t> *)j.xs, (Const<uint32_t> *)j.zs, (Const<T> *)j.cf, 0, 0, j.n_strings, 0,
         int(j.accumulate));
 }
 

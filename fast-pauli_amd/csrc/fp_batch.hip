@@ -386,7 +386,8 @@ fp_status build(fp_hip_batch *b, hipStream_t stream, bool columns)
             column_entries.push_back(fprt::ColumnEntry{
                 uint32_t(o->n_qubits), uint32_t(o->n_strings), e.dtype != FP_C128, e.accumulate != 0, e.n_states,
                 reinterpret_cast<uintptr_t>(e.states), reinterpret_cast<uintptr_t>(e.out),
-                reinterpret_cast<uintptr_t>(o->d_xz), reinterpret_cast<uintptr_t>(op.cf)});
+                reinterpret_cast<uintptr_t>(o->d_x32), reinterpret_cast<uintptr_t>(o->d_z32),
+                reinterpret_cast<uintptr_t>(op.cf)});
             // inputs read, columns written and read, outputs likewise (read first when accumulating)
             b->plan_bytes += double(entry_in_bytes(e)) * (e.accumulate ? 9.0 : 6.0);
             op.sshift = 64u;

@@ -218,11 +218,11 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
 namespace
 {
 
-// Configurations of k_apply_columns: one row a thread and four strings in flight, straight from
-// the column; or 2^13-row tiles in LDS, eight rows a thread.
+// Configurations of k_apply_columns: one row a thread and four or eight partner rows in flight,
+// straight from the column; or 2^13-row tiles in LDS, eight rows a thread.
 template <class T, int NS, bool WTD>
 fp_status launch_apply_columns(void const *cols, void *out, uint32_t n, uint32_t n_cols, uint32_t n_states,
-                               fpc::XZ const *xz, T const *cf, uint64_t cf_stride, uint32_t n_strings, uint32_t shift,
+                               uint32_t const *xs, uint32_t const *zs, T const *cf, uint64_t cf_stride, uint32_t n_strings, uint32_t shift,
                                int accumulate, bool lds, hipStream_t st)
 {
     typedef typename fpk::VecOf<T, NS>::type V;
@@ -231,7 +231,10 @@ fp_status launch_apply_columns(void const *cols, void *out, uint32_t n, uint32_t
         constexpr bool LDS = decltype(lds_tag)::value;
         constexpr uint32_t kTile = 6u + fpc::log2c(E) + fpc::log2c(TH / 64);
         constexpr size_t kLds = LDS ? sizeof(V) * E * TH : 0;
-        auto const kfn = &fpc::k_apply_columns<T, NS, E, U, TH, LDS, !LDS, WTD>;
+        // rows in flight: complex128 one batch ahead, complex64, whose terms take half the time, two
+        // (n = 16, one state, 500 strings: 20.1 us with one, 17.7 with two; complex128 19.3 / 23.2)
+        constexpr int D = LDS ? 1 : sizeof(T) == 4 && !WTD ? 3 : 2;
+        auto const kfn = &fpc::k_apply_columns<T, NS, E, U, TH, LDS, D, WTD>;
         if constexpr (LDS)
         {
             static std::once_flag once;
@@ -246,7 +249,7 @@ fp_status launch_apply_columns(void const *cols, void *out, uint32_t n, uint32_t
         uint32_t const tiles = n > kTile ? 1u << (n - kTile) : 1u, per = n < kTile ? 1u << (kTile - n) : 1u;
         uint32_t const groups = (n_cols + per - 1) / per;
         hipLaunchKernelGGL(kfn, dim3(tiles * groups), dim3(TH), kLds, st, static_cast<V const *>(cols),
-                           static_cast<V *>(out), n, n_cols, groups, tiles, xz, cf, cf_stride, n_states, n_strings,
+                           static_cast<V *>(out), n, n_cols, groups, tiles, xs, zs, cf, cf_stride, n_states, n_strings,
                            shift, accumulate);
         FP_LAUNCHED();
         return FP_OK;
@@ -279,8 +282,8 @@ bool apply_lds_tiles(uint32_t n, uint64_t n_cols)
 //  1: a power-of-two state count (weighted: one state, whose weights are then one row) and a
 //     batch of at most 8 MiB (one state: 32 MiB), which the L2s and the Infinity Cache serve;
 //     beyond 4 MiB from 64 strings (n = 20, one complex128 state: N = 24 41.6 us streaming /
-//     45.9, N = 64 113 / 112).  us, streaming / column: n = 10, 128 states, 64 strings 14.1 / 7.4;
-//     n = 18, one state, 1000 strings 286 / 148.
+//     45.9, N = 64 113 / 112).  us, streaming / column: n = 10, 128 states, 64 strings 14.1 / 6.9;
+//     n = 18, one state, 1000 strings 286 / 135.
 //  2: columns of at most 4 MiB (an XCD's L2), 8 MiB where the state count is not a power of two
 //     (the coset-tiled kernel is then at its slowest); enough work to pay the two transposed
 //     copies: from 32 strings and 3e7 (string, element) terms.  us, streaming or tiled / columns:
@@ -323,7 +326,7 @@ fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void con
         return FP_OK;
     uint32_t const n = uint32_t(ops->n_qubits), N = uint32_t(ops->n_strings);
     size_t const esz = c64 ? 8 : 16;
-    auto const *xz = ops->d_xz;
+    uint32_t const *xs = ops->d_x32, *zs = ops->d_z32;
     bool const aligned16 = ((reinterpret_cast<uintptr_t>(states) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
     // scratch: [transposed states | transposed outputs | weights]
     bool const pairs = c64 && n <= 18 && n_states > 1;
@@ -373,10 +376,10 @@ fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void con
             bool const two = c64 && shift > 0 && aligned16 && dim * n_states >= (size_t(1) << 19);
             if constexpr (sizeof(T) == 4)
                 if (two)
-                    return launch_apply_columns<T, 2, false>(states, out, n + shift - 1, 1, 1, xz, coef, 0, N,
+                    return launch_apply_columns<T, 2, false>(states, out, n + shift - 1, 1, 1, xs, zs, coef, 0, N,
                                                              shift - 1, accumulate, false, st);
-            return weighted ? launch_apply_columns<T, 1, true>(states, out, n, 1, 1, xz, w, N, N, 0, accumulate, false, st)
-                            : launch_apply_columns<T, 1, false>(states, out, n + shift, 1, 1, xz, coef, 0, N, shift,
+            return weighted ? launch_apply_columns<T, 1, true>(states, out, n, 1, 1, xs, zs, w, N, N, 0, accumulate, false, st)
+                            : launch_apply_columns<T, 1, false>(states, out, n + shift, 1, 1, xs, zs, coef, 0, N, shift,
                                                                 accumulate, false, st);
         }
         auto slabs = [&](auto ns_tag) -> fp_status {
@@ -394,9 +397,9 @@ fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void con
                 FP_LAUNCHED();
                 bool const lds = apply_lds_tiles(n, nc);
                 fp_status const s =
-                    weighted ? launch_apply_columns<T, NS, true>(ic, oc, n, nc, nst, xz, w + 2 * c0 * N, N, N, 0,
+                    weighted ? launch_apply_columns<T, NS, true>(ic, oc, n, nc, nst, xs, zs, w + 2 * c0 * N, N, N, 0,
                                                                  accumulate, lds, st)
-                             : launch_apply_columns<T, NS, false>(ic, oc, n, nc, nst, xz, coef, 0, N, 0, accumulate,
+                             : launch_apply_columns<T, NS, false>(ic, oc, n, nc, nst, xs, zs, coef, 0, N, 0, accumulate,
                                                                   lds, st);
                 if (s != FP_OK)
                     return s;

@@ -141,7 +141,7 @@ void free_device(fp_hip_ops *o)
     o->d_arena = nullptr;
     o->arena_bytes = 0;
     o->d_x = o->d_z = nullptr;
-    o->d_xz = nullptr;
+    o->d_x32 = o->d_z32 = nullptr;
     o->d_meta = nullptr;
     o->d_ny = nullptr;
     o->d_cf128 = o->d_scale = o->d_kappa_c = o->d_kappa = o->d_rowsum128 = o->d_wr64 = o->d_wi64 = nullptr;
@@ -205,11 +205,11 @@ template <class T> fp_status upload(T **dptr, std::vector<T> const &h)
     return FP_OK;
 }
 
-// Arena layout: xz | x | z | ny | meta | cf128 | cf64 | scale | kappa_c | kappa,
+// Arena layout: x32 | z32 | x | z | ny | meta | cf128 | cf64 | scale | kappa_c | kappa,
 // each section 256-byte aligned.
 struct ArenaLayout
 {
-    size_t xz, x, z, ny, meta, cf128, cf64, scale, kappa_c, kappa, ev_chunks, ev_strs, total;
+    size_t x32, z32, x, z, ny, meta, cf128, cf64, scale, kappa_c, kappa, ev_chunks, ev_strs, total;
 };
 
 ArenaLayout arena_layout(size_t N)
@@ -217,8 +217,9 @@ ArenaLayout arena_layout(size_t N)
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     ArenaLayout L{};
     size_t off = 0;
-    // (the apply kernel on columns reads kXzPad records past the end of xz, cf128 and cf64)
-    L.xz = off, off += up((N + fpc::kXzPad) * sizeof(fpc::XZ));
+    // (the apply kernel on columns reads kXzPad records past the end of x32, z32, cf128 and cf64)
+    L.x32 = off, off += up((N + fpc::kXzPad) * sizeof(uint32_t));
+    L.z32 = off, off += up((N + fpc::kXzPad) * sizeof(uint32_t));
     L.x = off, off += up(N * sizeof(uint64_t));
     L.z = off, off += up(N * sizeof(uint64_t));
     L.ny = off, off += up(N * sizeof(uint32_t));
@@ -390,7 +391,8 @@ fp_status ops_assign(fp_hip_ops *o, size_t n_qubits, size_t n_strings, uint8_t c
         o->ny[s] = ny;
         uint32_t const hb = x ? 63u - uint32_t(__builtin_clzll(x)) : 0u;
         uint32_t const mode = x == 0 ? fpk::kModeSelf : ((ny & 1u) ? fpk::kModeIm : fpk::kModeRe);
-        at<fpc::XZ>(h, L.xz)[s] = fpc::XZ{uint32_t(x), uint32_t(z)};
+        at<uint32_t>(h, L.x32)[s] = uint32_t(x);
+        at<uint32_t>(h, L.z32)[s] = uint32_t(z);
         at<uint64_t>(h, L.x)[s] = x;
         at<uint64_t>(h, L.z)[s] = z;
         at<uint32_t>(h, L.ny)[s] = ny;
@@ -413,7 +415,8 @@ fp_status ops_assign(fp_hip_ops *o, size_t n_qubits, size_t n_strings, uint8_t c
         o->arena_bytes = L.total;
     }
     void *d = o->d_arena;
-    o->d_xz = at<fpc::XZ>(d, L.xz);
+    o->d_x32 = at<uint32_t>(d, L.x32);
+    o->d_z32 = at<uint32_t>(d, L.z32);
     o->d_x = at<uint64_t>(d, L.x);
     o->d_z = at<uint64_t>(d, L.z);
     o->d_ny = at<uint32_t>(d, L.ny);

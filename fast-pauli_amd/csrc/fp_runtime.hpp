@@ -259,7 +259,7 @@ struct fp_hip_ops
     // device copies (pointers into the arena)
     uint64_t *d_x = nullptr, *d_z = nullptr;
     fpk::StringMeta *d_meta = nullptr;
-    fpc::XZ *d_xz = nullptr;     // x and z in 32 bits (n <= 32), read kXzPad records past the end
+    uint32_t *d_x32 = nullptr, *d_z32 = nullptr; // x and z in 32 bits, read kXzPad past the end
     double *d_cf128 = nullptr;   // c_s * (-i)^{nY_s}, complex128
     float *d_cf64 = nullptr;     // same, complex64
     double *d_scale = nullptr;   // c_s * kappa_s (complex, FP64): PauliOp EV

@@ -234,17 +234,11 @@ struct ColStr
     double sim;
 };
 
-// One string's masks (n <= 32), for the apply kernel on columns.
-struct XZ
-{
-    uint32_t x, z;
-};
-
 // Many operators on the columns of one slab (k_apply_columns_batch, k_columns_batch).
 struct ColJob
 {
     uint64_t cols;   // byte offset of the first column in both slabs
-    uint64_t xz, cf; // device addresses of the operator's XZ records and folded coefficients
+    uint64_t xs, zs, cf; // device addresses of the operator's masks and folded coefficients
     uint32_t n, n_cols, n_strings, accumulate;
 };
 // Blocks [block0, ...) of a job, from position `start` of an XCD's queue on.

@@ -769,7 +769,7 @@ void build_column_rounds(std::vector<ColumnEntry> const &entries, size_t slab_by
                 break;
             uint64_t const c0 = pairs ? 2 * done : done;
             uint64_t const ns = std::min<uint64_t>(pairs ? 2 * take : take, e.n_states - c0);
-            jobs.push_back(fpc::ColJob{at, e.xz, e.cf, e.n, uint32_t(take), e.n_strings, e.accumulate ? 1u : 0u});
+            jobs.push_back(fpc::ColJob{at, e.xs, e.zs, e.cf, e.n, uint32_t(take), e.n_strings, e.accumulate ? 1u : 0u});
             // blocks: the tiles of each column, or the groups of columns that fill a tile
             job_blocks.push_back(e.n > tile ? take << (e.n - tile)
                                             : (take + (uint64_t(1) << (tile - e.n)) - 1) >> (tile - e.n));

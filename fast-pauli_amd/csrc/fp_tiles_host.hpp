@@ -84,13 +84,13 @@ fp_status build_tile_image(StringTable const &st, int kind, uint32_t k, uint32_t
 fp_status build_column_image(StringTable const &st, bool c64, uint32_t per_item, TileImage &out);
 
 // An apply of a batch that runs on columns.  Addresses are device addresses: the states and
-// outputs, and the operator's fpc::XZ records and folded coefficients of its type.
+// outputs, and the operator's masks (32 bits) and folded coefficients of its type.
 struct ColumnEntry
 {
     uint32_t n, n_strings;
     bool c64, accumulate;
     uint64_t n_states;
-    uint64_t states, out, xz, cf;
+    uint64_t states, out, xs, zs, cf;
 };
 
 // The launches of one slab of columns: copies in, one apply kernel, copies out.

@@ -254,7 +254,7 @@ int check_rounds(std::vector<fprt::ColumnEntry> const &es, size_t slab)
         {
             fprt::ColumnEntry const &e = es[spans[j].entry];
             bad += jobs[j].cols != spans[j].at || jobs[j].n != e.n || jobs[j].n_strings != e.n_strings ||
-                   jobs[j].xz != e.xz || jobs[j].cf != e.cf || (jobs[j].accumulate != 0) != e.accumulate ||
+                   jobs[j].xs != e.xs || jobs[j].zs != e.zs || jobs[j].cf != e.cf || (jobs[j].accumulate != 0) != e.accumulate ||
                    jobs[j].n_cols * (row << e.n) != spans[j].size;
             uint64_t const per = e.n < tile ? 1u << (tile - e.n) : 1u, tiles = e.n > tile ? 1u << (e.n - tile) : 1u;
             hit[j].assign((jobs[j].n_cols + per - 1) / per * tiles, 0);
@@ -296,7 +296,8 @@ int round_cases(Rng &r)
                     e.n_states = 1 + r.next() % (count > 9 ? 9 : 70);
                     e.states = 0x1000 * (4 * i + 1);
                     e.out = 0x1000 * (4 * i + 2);
-                    e.xz = 0x1000 * (4 * i + 3);
+                    e.xs = 0x1000 * (4 * i + 3);
+                    e.zs = e.xs + 0x800;
                     e.cf = 0x1000 * (4 * i + 4);
                     es.push_back(e);
                 }
