@@ -185,12 +185,17 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
     uint32_t const g = (item.p << kWaveBits) | wave; // row bits above the slots
     uint32_t const la = (wave << 13) | (lane << 4);
     double acc_re = 0.0, acc_im = 0.0;
+    // An entry's partner rows are asked for before the barrier that ends the previous one, and
+    // its first records with them: a wave that is done early waits for its loads meanwhile.
+    ColEntry next = entries[item.entry_first];
+    ColStr first = strs[next.first];
     for (uint32_t e = 0; e < item.entry_count; ++e)
     {
-        ColEntry const en = entries[item.entry_first + e];
-        __syncthreads(); // the previous partner tile is no longer read
+        ColEntry const en = next;
+        ColStr st = first;
         if (en.u == 0)
         {
+            __syncthreads(); // the previous partner tile is no longer read
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 tile[e0 + uint32_t(i) * 64u] = L[i];
@@ -202,10 +207,13 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 r[i] = src[uint32_t(i) * 64u];
+            __syncthreads();
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 tile[e0 + uint32_t(i) * 64u] = r[i];
         }
+        next = entries[item.entry_first + (e + 1 < item.entry_count ? e + 1 : e)];
+        first = strs[next.first];
         __syncthreads();
         uint32_t const end = en.first + en.count;
         for (uint32_t s = en.first; s < end;)
@@ -213,7 +221,6 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
             // strings of one case follow each other: one branch to their body, which then
             // runs the whole stretch with the next record in flight (a branch per string:
             // 2174 us instead of 1603 at n = 14, 1024 strings, 1000 complex128 states)
-            ColStr st = strs[s];
             uint32_t const stretch = st.code >> kColRunShift;
             uint32_t const stop = stretch < end - s ? s + stretch : end;
             auto signs = [&](ColStr const &r, T(&sg)[3], T &s0) {
@@ -241,7 +248,8 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
                     // columns gain 2 %, n = 14 nothing)
                     for (; s + 1 < stop; s += 2)
                     {
-                        ColStr const a = strs[s], b = strs[s + 1];
+                        ColStr const a = st, b = strs[s + 1];
+                        st = strs[s + 2]; // one record follows the last
                         P Ra[8], Rb[8];
                         load_partners<T, XS, HALF>(Ra, smem + (la ^ a.px));
                         load_partners<T, XS, HALF>(Rb, smem + (la ^ b.px));
@@ -253,19 +261,18 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
                     }
                     if (s >= stop)
                         return;
-                    st = strs[s];
                 }
                 while (true)
                 {
-                    ColStr const nx = strs[s + 1]; // one record follows the last
+                    ColStr const nx = strs[s + 1];
                     P R[8];
                     load_partners<T, XS, HALF>(R, smem + (la ^ st.px));
                     T sg[3], s0;
                     signs(st, sg, s0);
                     add(st, pair_sum<T, XS, SUB, IM, HALF>(L, R, sg, s0));
+                    st = nx;
                     if (++s >= stop)
                         break;
-                    st = nx;
                 }
             };
 #define FP_COL_CASE(XS, SUB, IM, HALF)                                                                                 \
@@ -294,10 +301,11 @@ __global__ __launch_bounds__(kThreads, 4) void k_ev_columns(typename Piece<T>::t
             {
                 for (; s < stop; ++s)
                 {
-                    st = strs[s];
+                    ColStr const nx = strs[s + 1];
                     T sg[3], s0;
                     signs(st, sg, s0);
                     add(st, self_sum<T>(L, sg, s0));
+                    st = nx;
                 }
             }
             else if constexpr (kC64)

@@ -12,6 +12,7 @@
 #include "fp_tiles_host.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <utility>
@@ -655,21 +656,30 @@ fp_status build_column_image(StringTable const &st, bool c64, uint32_t per_item,
     }
     strs.push_back(fpc::ColStr{}); // read ahead of the last string
     uint64_t const tiles = n > w ? uint64_t(1) << (n - w) : 1u;
-    double const limit = std::max<uint32_t>(per_item, 1);
     for (uint64_t p = 0; p < tiles; ++p)
     {
-        double cost = limit; // the first entry opens an item
+        auto leads = [&](ColClass const &cl) { return !cl.u || !((p >> cl.lead) & 1u); };
+        // equal items, not full ones and a rest: their blocks end together (n = 14, 1024 strings,
+        // 200 complex128 states: 371 us with a rest of a third, now 329)
+        double total = 0.0;
+        for (ColClass const &cl : classes)
+            if (leads(cl))
+                for (fpc::ColStr const &r : cl.strs)
+                    total += record_cost(r);
+        double const n_items = std::max(1.0, std::ceil(total / std::max<uint32_t>(per_item, 1)));
+        double cost = 0.0, limit = 0.0, cut = 0.0; // the first entry opens an item
         for (size_t c = 0; c < classes.size(); ++c)
         {
             ColClass const &cl = classes[c];
-            if (cl.u && ((p >> cl.lead) & 1u))
+            if (!leads(cl))
                 continue;
             for (size_t i = 0; i < cl.strs.size();)
             {
                 if (cost >= limit)
                 {
                     items.push_back(fpc::ColItem{uint32_t(p), uint32_t(entries.size()), 0, 0});
-                    cost = 0.0;
+                    cut += 1.0;
+                    limit = cut < n_items ? total * cut / n_items : total + 1.0;
                 }
                 size_t j = i;
                 while (j < cl.strs.size() && cost < limit)
