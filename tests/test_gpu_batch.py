@@ -372,3 +372,26 @@ def test_column_entries_bit_exact(hip, graph):
         for e in entries:
             check(e, e.result())
     b.destroy()
+
+
+def test_column_launches_on_two_streams(hip):
+    """Launches of one batch on two streams share its column buffers: the later one waits."""
+    H.say("batch columns on two streams")
+    entries = [Entry(_abi.FP_BATCH_APPLY, 14, 64, 33, C64, False, seed=80),
+               Entry(_abi.FP_BATCH_APPLY, 15, 64, 40, C64, False, seed=81)]
+    refs = [e.alone() for e in entries]
+    b = Batch()
+    for e in entries:
+        b.add(e.kind, e.ops, e.d_in.ptr, e.d_out.ptr, 1 << e.n, e.S, e.dtype, e.accumulate)
+    streams = [_abi.Stream(), _abi.Stream()]
+    b.launch(streams[0])
+    for i in range(1, 8):
+        b.launch(streams[i % 2])
+    for s in streams:
+        s.synchronize()
+    assert b.info()["column_entries"] == 2
+    for e, r in zip(entries, refs):
+        assert np.array_equal(e.result(), r)
+    b.destroy()
+    for s in streams:
+        s.destroy()
