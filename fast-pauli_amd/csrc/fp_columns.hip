@@ -295,6 +295,10 @@ bool apply_lds_tiles(uint32_t n, uint64_t n_cols)
 //     n = 14, 1000 complex128 states, 500 strings 8500 / 3270; n = 20, 19 complex64 states, 512
 //     strings 10900 / 5710; but n = 12, 100 complex64 states, 64 strings (2.6e7 terms) 16.2 / 21.3
 //     and n = 20, 16 complex64 states, 64 strings 619 / 733.
+//     Weighted, whose row-major form reads a weight per string and element: also from 48 strings
+//     on fewer than 2^19 elements.  n = 10, 2 states, 89 strings 43.8 / 17.2; n = 12, 100 states, 48
+//     strings 42.7 / 36.7; n = 9, 50 states, 200 strings 122 / 45; but n = 9, 2 states, 32 strings,
+//     200 operators 37.7 / 49.7 and n = 18, 2 states, 40 strings 30.4 / 42.2.
 // FAST_PAULI_APPLY_KERNEL=columns forces 1 or 2 where the shape allows, other values forbid them.
 int apply_columns_route(fp_hip_ops const *ops, int dtype, size_t n_states, bool weighted)
 {
@@ -318,6 +322,8 @@ int apply_columns_route(fp_hip_ops const *ops, int dtype, size_t n_states, bool 
         return 2;
     if (col_bytes > (size_t(4) << 20) && pow2)
         return 0;
+    if (weighted && N >= 48 && elements < (size_t(1) << 19))
+        return 2;
     return N >= 32 && double(N) * double(elements) >= 3e7 ? 2 : 0;
 }
 

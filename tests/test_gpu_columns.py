@@ -194,5 +194,9 @@ def test_apply_columns_rule(hip, monkeypatch):
                           (20, 24, 1, False), (21, 96, 8, False), (10, 1, 128, False)):
         ops = _abi.Ops(syn.random_codes(N, n, seed=n))
         assert _abi.op_apply_columns(ops, C128, 1 << n, S) == want, (n, N, S)
+    # weights per state: from 48 strings on small batches too
+    for n, N, S, want in ((10, 48, 2, True), (10, 47, 2, False), (18, 48, 2, False), (18, 48, 3, True)):
+        ops = _abi.Ops(syn.random_codes(N, n, seed=n))
+        assert _abi.op_apply_columns(ops, C128, 1 << n, S, weighted=True) == want, (n, N, S)
     monkeypatch.setenv("FAST_PAULI_APPLY_KERNEL", "tiled")
     assert not _abi.op_apply_columns(_abi.Ops(syn.random_codes(64, 10, seed=1)), C128, 1 << 10, 128)
