@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -17,6 +18,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <tuple>
 #include <type_traits>
 #include <vector>
 
@@ -32,24 +34,86 @@ namespace fprt
 // Per-stream scratch: reduction partials etc.  Grown on demand (after the
 // stream has drained), never shrunk.  Calls on one stream are ordered, and the
 // entry points that use scratch hold the stream's StreamGuard until their
-// kernels are enqueued, so one buffer per stream suffices.
+// kernels are enqueued, so one buffer per stream suffices.  "Stream" is the
+// stream, not its handle: see StreamKey.
 // ---------------------------------------------------------------------------
 struct Scratch
 {
     void *ptr = nullptr;
     size_t bytes = 0;
 };
+
+// A stream's scratch and guard are found by its handle.  hipStreamPerThread is one handle for a
+// stream of each host thread: there a number of the thread, never used again, tells them apart.
+struct StreamKey
+{
+    int dev;
+    hipStream_t stream;
+    uint64_t thread;
+    bool operator<(StreamKey const &o) const
+    {
+        return std::tie(dev, stream, thread) < std::tie(o.dev, o.stream, o.thread);
+    }
+};
 std::mutex g_scratch_mu;
-std::map<std::pair<int, hipStream_t>, Scratch> g_scratch;
-std::map<std::pair<int, hipStream_t>, std::unique_ptr<std::recursive_mutex>> g_stream_mu;
+std::map<StreamKey, Scratch> g_scratch;
+std::map<StreamKey, std::unique_ptr<std::recursive_mutex>> g_stream_mu;
+
+namespace
+{
+
+// Frees the scratch of the streams that `match` (g_scratch_mu held; their work has ended, or
+// hipFree waits for it).
+template <class F> void drop_scratch(F match)
+{
+    for (auto it = g_scratch.begin(); it != g_scratch.end();)
+    {
+        if (match(it->first))
+        {
+            (void)hipFree(it->second.ptr);
+            it = g_scratch.erase(it);
+        }
+        else
+            ++it;
+    }
+}
+
+// The calling thread's number; its per-thread stream's scratch goes with the thread.
+struct ThreadNumber
+{
+    uint64_t value;
+    ThreadNumber()
+    {
+        static std::atomic<uint64_t> next{1};
+        value = next++;
+    }
+    ~ThreadNumber()
+    {
+        std::lock_guard<std::mutex> lock(g_scratch_mu);
+        drop_scratch([this](StreamKey const &k) { return k.thread == value; });
+        for (auto it = g_stream_mu.begin(); it != g_stream_mu.end();)
+            it = it->first.thread == value ? g_stream_mu.erase(it) : std::next(it);
+    }
+};
+
+StreamKey stream_key(int dev, hipStream_t stream)
+{
+    if (stream != hipStreamPerThread)
+        return StreamKey{dev, stream, 0};
+    static thread_local ThreadNumber number;
+    return StreamKey{dev, stream, number.value};
+}
+
+} // namespace
 
 StreamGuard::StreamGuard(hipStream_t stream)
 {
     int dev = 0;
     (void)hipGetDevice(&dev);
+    StreamKey const key = stream_key(dev, stream);
     {
         std::lock_guard<std::mutex> lock(g_scratch_mu);
-        auto &m = g_stream_mu[{dev, stream}];
+        auto &m = g_stream_mu[key];
         if (!m)
             m = std::make_unique<std::recursive_mutex>();
         mu_ = m.get();
@@ -66,8 +130,9 @@ fp_status scratch_get(hipStream_t stream, size_t bytes, void **out)
 {
     int dev = 0;
     FP_HIP(hipGetDevice(&dev));
+    StreamKey const key = stream_key(dev, stream);
     std::lock_guard<std::mutex> lock(g_scratch_mu);
-    Scratch &s = g_scratch[{dev, stream}];
+    Scratch &s = g_scratch[key];
     if (s.bytes < bytes)
     {
         if (s.ptr)
@@ -898,16 +963,8 @@ fp_status fp_hip_stream_destroy(void *stream)
     FP_HIP(hipStreamSynchronize(s));
     {
         std::lock_guard<std::mutex> lock(g_scratch_mu);
-        for (auto it = g_scratch.begin(); it != g_scratch.end();)
-        {
-            if (it->first.second == s)
-            {
-                (void)hipFree(it->second.ptr);
-                it = g_scratch.erase(it);
-            }
-            else
-                ++it;
-        }
+        uint64_t const thread = stream_key(0, s).thread;
+        drop_scratch([&](StreamKey const &k) { return k.stream == s && k.thread == thread; });
     }
     FP_HIP(hipStreamDestroy(s));
     return FP_OK;

@@ -25,8 +25,10 @@
  *    the output (out += result, the reference C++ API's semantics); 0
  *    overwrites it (what the reference's Python layer gets from its fresh,
  *    zeroed outputs).
- *  - Library-owned scratch (reduction partials) is kept per stream.  Calls
- *    on one stream are ordered; calls on different streams may overlap.
+ *  - Library-owned scratch (reduction partials, transposed states) is kept per
+ *    stream.  Calls on one stream are ordered; calls on different streams may
+ *    overlap.  hipStreamPerThread counts as one stream for each host thread; its
+ *    scratch is freed when the thread ends.
  */
 #ifndef FAST_PAULI_HIP_H
 #define FAST_PAULI_HIP_H

@@ -6,6 +6,8 @@ structured string sets.
 Bars, as for the other kernels: complex128 within 1e-12, complex64 (FP32 products, FP64 sums)
 within 1e-5 of the FP64 oracle."""
 
+import threading
+
 import numpy as np
 import pytest
 
@@ -200,3 +202,48 @@ def test_apply_columns_rule(hip, monkeypatch):
         assert _abi.op_apply_columns(ops, C128, 1 << n, S, weighted=True) == want, (n, N, S)
     monkeypatch.setenv("FAST_PAULI_APPLY_KERNEL", "tiled")
     assert not _abi.op_apply_columns(_abi.Ops(syn.random_codes(64, 10, seed=1)), C128, 1 << 10, 128)
+
+
+# ---------------------------------------------------------------------------
+# streams, threads and captured graphs
+# ---------------------------------------------------------------------------
+PER_THREAD = 2  # the handle hipStreamPerThread: another stream in every host thread
+
+
+def test_columns_on_per_thread_streams(hip):
+    """One handle, two host threads, two streams: the transposed slabs (and partials) are each
+    thread's own.  Applies IEEE-equal, expectation values identical, to the null stream's."""
+    H.say("columns on per-thread streams")
+    n, N, S, rounds = 15, 64, 45, 12  # 23 MB of columns: the threads' kernels overlap
+    work = []
+    for seed in (1, 2):
+        ops = _abi.Ops(syn.random_codes(N, n, seed=seed), syn.random_coeffs(N, seed=seed))
+        assert _abi.op_apply_columns(ops, C128, 1 << n, S)
+        psi = syn.random_states(1 << n, S, seed=seed)
+        want = H.op_apply(ops, psi, C128), H.op_expectation(ops, psi, C128)
+        outs = [_abi.DeviceBuffer(psi.nbytes) for _ in range(rounds)]
+        evs = [_abi.DeviceBuffer(S * 16) for _ in range(rounds)]
+        work.append((ops, _abi.DeviceBuffer.from_array(psi), outs, evs, want, psi.shape))
+    _abi.synchronize()
+    failed, go = [], threading.Barrier(2)
+
+    def body(ops, d_in, outs, evs, *_):
+        try:
+            go.wait(timeout=30)
+            for d_out, d_ev in zip(outs, evs):
+                _abi.call("fp_hip_op_apply", ops.handle, C128, d_in.ptr, d_out.ptr, 1 << n, S, 0, PER_THREAD)
+                _abi.call("fp_hip_op_expectation", ops.handle, C128, d_in.ptr, d_ev.ptr, 1 << n, S, 0, PER_THREAD)
+            _abi.call("fp_hip_stream_synchronize", PER_THREAD)
+        except Exception as e:  # reported by the main thread
+            failed.append(e)
+
+    threads = [threading.Thread(target=body, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    for _, _, outs, evs, (apply, ev), shape in work:
+        for d_out, d_ev in zip(outs, evs):
+            assert np.array_equal(d_out.to_array(np.complex128, shape), apply)
+            assert np.array_equal(d_ev.to_array(np.complex128, (S,)), ev)
