@@ -30,17 +30,6 @@ size_t round256(size_t v)
     return (v + 255) / 256 * 256;
 }
 
-bool capturing(hipStream_t st)
-{
-    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &s) != hipSuccess)
-    {
-        (void)hipGetLastError();
-        return true;
-    }
-    return s != hipStreamCaptureStatusNone;
-}
-
 // Columns per tile of the expectation kernel and columns per slab.
 struct ColGeom
 {
@@ -110,7 +99,7 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
 {
     *done = false;
     bool const c64 = dtype != FP_C128;
-    if (!ws && capturing(st)) // the slab may have to be allocated
+    if (!ws && stream_capturing(st)) // the slab may have to be allocated
         return FP_OK;
     // one aligned state is a column already
     bool const in_place = n_states == 1 && (reinterpret_cast<uintptr_t>(states) & 15u) == 0;
@@ -333,7 +322,7 @@ fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void con
     *done = false;
     bool const weighted = kind == kTilesWeightedApply, c64 = dtype != FP_C128;
     int const route = apply_columns_route(ops, dtype, n_states, weighted);
-    if (route == 0 || (route == 2 || weighted ? capturing(st) : false))
+    if (route == 0 || ((route == 2 || weighted) && stream_capturing(st)))
         return FP_OK;
     uint32_t const n = uint32_t(ops->n_qubits), N = uint32_t(ops->n_strings);
     size_t const esz = c64 ? 8 : 16;

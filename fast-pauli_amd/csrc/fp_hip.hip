@@ -31,8 +31,8 @@ namespace fprt
 {
 
 // ---------------------------------------------------------------------------
-// Per-stream scratch: reduction partials etc.  Grown on demand (after the
-// stream has drained), never shrunk.  Calls on one stream are ordered, and the
+// Per-stream scratch: reduction partials, transposed states etc.  Grown on demand
+// (after the stream has drained), never shrunk.  Calls on one stream are ordered, and the
 // entry points that use scratch hold the stream's StreamGuard until their
 // kernels are enqueued, so one buffer per stream suffices.  "Stream" is the
 // stream, not its handle: see StreamKey.
@@ -41,6 +41,8 @@ struct Scratch
 {
     void *ptr = nullptr;
     size_t bytes = 0;
+    bool captured = false;       // kernels in a graph hold its address: outgrown, it is kept
+    std::vector<void *> outgrown; // until the stream goes
 };
 
 // A stream's scratch and guard are found by its handle.  hipStreamPerThread is one handle for a
@@ -70,6 +72,8 @@ template <class F> void drop_scratch(F match)
     {
         if (match(it->first))
         {
+            for (void *p : it->second.outgrown)
+                (void)hipFree(p);
             (void)hipFree(it->second.ptr);
             it = g_scratch.erase(it);
         }
@@ -106,6 +110,17 @@ StreamKey stream_key(int dev, hipStream_t stream)
 
 } // namespace
 
+bool stream_capturing(hipStream_t stream)
+{
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &s) != hipSuccess)
+    {
+        (void)hipGetLastError(); // (the null stream beside another stream's capture)
+        return false;
+    }
+    return s != hipStreamCaptureStatusNone;
+}
+
 StreamGuard::StreamGuard(hipStream_t stream)
 {
     int dev = 0;
@@ -133,21 +148,44 @@ fp_status scratch_get(hipStream_t stream, size_t bytes, void **out)
     StreamKey const key = stream_key(dev, stream);
     std::lock_guard<std::mutex> lock(g_scratch_mu);
     Scratch &s = g_scratch[key];
+    bool const capture = stream_capturing(stream);
     if (s.bytes < bytes)
     {
-        if (s.ptr)
+        size_t want = std::max<size_t>(bytes, size_t(1) << 20);
+        if (s.ptr && (s.captured || capture))
         {
-            // earlier calls on this stream have enqueued all their kernels (the
-            // caller holds the stream's guard): once they finish, the buffer is free
-            FP_HIP(hipStreamSynchronize(stream));
-            FP_HIP(hipFree(s.ptr));
-            s.ptr = nullptr;
-            s.bytes = 0;
+            // graphs captured on this stream use the old buffer (or this capture forbids waiting
+            // for its kernels): it stays, and twice its size, where there is room for it, bounds
+            // the sum of what is kept
+            void *ptr = nullptr;
+            size_t const twice = std::max(want, 2 * s.bytes);
+            if (hipMalloc(&ptr, twice) == hipSuccess)
+                want = twice;
+            else
+            {
+                (void)hipGetLastError();
+                FP_HIP(hipMalloc(&ptr, want));
+            }
+            s.outgrown.push_back(s.ptr);
+            s.ptr = ptr;
         }
-        size_t const want = std::max<size_t>(bytes, size_t(1) << 20);
-        FP_HIP(hipMalloc(&s.ptr, want));
+        else
+        {
+            if (s.ptr)
+            {
+                // earlier calls on this stream have enqueued all their kernels (the
+                // caller holds the stream's guard): once they finish, the buffer is free
+                FP_HIP(hipStreamSynchronize(stream));
+                FP_HIP(hipFree(s.ptr));
+                s.ptr = nullptr;
+                s.bytes = 0;
+            }
+            FP_HIP(hipMalloc(&s.ptr, want));
+        }
         s.bytes = want;
+        s.captured = false;
     }
+    s.captured = s.captured || capture;
     *out = s.ptr;
     return FP_OK;
 }

@@ -24,8 +24,12 @@
 namespace fprt
 {
 
+// Whether work on `stream` is being captured into a graph.
+bool stream_capturing(hipStream_t stream);
+
 // Per-stream device scratch of at least `bytes`; the pointer stays valid until
-// the next, larger request on the same stream.  Callers hold a StreamGuard for
+// the next, larger request on the same stream, or, handed out while the stream is
+// captured, until the stream is destroyed.  Callers hold a StreamGuard for
 // the stream until the kernels that use the buffer are enqueued.
 fp_status scratch_get(hipStream_t stream, size_t bytes, void **out);
 

@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import ctypes
 import sys
 
 import numpy as np
@@ -113,3 +114,28 @@ def ev_scaled_err(got, ref, coeffs, psi) -> float:
     scale = np.abs(np.asarray(coeffs)).sum() * (np.abs(np.asarray(psi, np.complex128)) ** 2).sum(axis=0)
     d = np.abs(np.asarray(got, np.complex128) - np.asarray(ref, np.complex128))
     return float((d / scale).max())
+
+
+class Graph:
+    """What `fn(stream)` enqueues on `stream` while it is captured, to be replayed there."""
+
+    def __init__(self, stream, fn, mode: int = 0):
+        lib, vp = _abi.lib(), ctypes.c_void_p
+        self.stream, self.graph, self.exec = stream, vp(), vp()
+        assert lib.hipStreamBeginCapture(vp(stream.handle), mode) == 0
+        try:
+            fn(stream.handle)
+        finally:
+            ended = lib.hipStreamEndCapture(vp(stream.handle), ctypes.byref(self.graph))
+        assert ended == 0, ended
+        assert lib.hipGraphInstantiate(ctypes.byref(self.exec), self.graph, None, None, ctypes.c_size_t(0)) == 0
+
+    def replay(self) -> None:
+        assert _abi.lib().hipGraphLaunch(self.exec, ctypes.c_void_p(self.stream.handle)) == 0
+        self.stream.synchronize()
+
+    def destroy(self) -> None:
+        for name, h in (("hipGraphExecDestroy", self.exec), ("hipGraphDestroy", self.graph)):
+            if h:
+                getattr(_abi.lib(), name)(h)
+        self.exec = self.graph = None

@@ -247,3 +247,36 @@ def test_columns_on_per_thread_streams(hip):
         for d_out, d_ev in zip(outs, evs):
             assert np.array_equal(d_out.to_array(np.complex128, shape), apply)
             assert np.array_equal(d_ev.to_array(np.complex128, (S,)), ev)
+
+
+def test_captured_scratch_outlives_larger_calls(hip, monkeypatch):
+    """A graph holds the scratch its stream had at the capture: an apply on columns, which needs
+    more, takes another buffer.  Replays, with eager work between them, equal the eager call."""
+    H.say("captured expectation beside larger applies")
+    stream = _abi.Stream()
+    n, N, S = 10, 12, 5
+    ops = _abi.Ops(syn.random_codes(N, n, seed=3), syn.random_coeffs(N, seed=3))
+    psi = syn.random_states(1 << n, S, seed=3)
+    d_in, d_out = _abi.DeviceBuffer.from_array(psi), _abi.DeviceBuffer(S * 16)
+
+    def expect(handle):
+        _abi.call("fp_hip_op_expectation", ops.handle, C128, d_in.ptr, d_out.ptr, 1 << n, S, 0, handle)
+
+    monkeypatch.setenv("FAST_PAULI_EV_KERNEL", "stream")
+    expect(stream.handle)
+    stream.synchronize()
+    want = d_out.to_array(np.complex128, (S,))
+    graph = H.Graph(stream, expect)
+    for m, T in ((13, 70), (14, 90), (15, 100)):  # scratch of 18, 47 and 105 MB
+        big = _abi.Ops(syn.random_codes(64, m, seed=m), syn.random_coeffs(64, seed=m))
+        phi = syn.random_states(1 << m, T, seed=m)
+        d_phi, d_big = _abi.DeviceBuffer.from_array(phi), _abi.DeviceBuffer(phi.nbytes)
+        assert _abi.op_apply_columns(big, C128, 1 << m, T)
+        _abi.call("fp_hip_op_apply", big.handle, C128, d_phi.ptr, d_big.ptr, 1 << m, T, 0, stream.handle)
+        d_out.zero()
+        _abi.synchronize()
+        graph.replay()
+        assert np.array_equal(d_out.to_array(np.complex128, (S,)), want)
+        assert np.array_equal(d_big.to_array(np.complex128, phi.shape), H.op_apply(big, phi, C128))
+    graph.destroy()
+    stream.destroy()
