@@ -72,6 +72,7 @@ struct fp_hip_batch
     {
         uint32_t entry;
         fprt::TileTables *tt;
+        fprt::TileAddr at;
         fprt::TileGeom geo;
     };
     std::vector<Split> split;
@@ -198,8 +199,8 @@ fp_status enqueue_kernels(fp_hip_batch *b, hipStream_t stream)
     for (fp_hip_batch::Split const &sp : b->split)
     {
         BatchEntry const &e = b->entries[sp.entry];
-        fp_status const r = fprt::launch_op_apply_tiled(sp.tt, sp.geo, e.dtype, e.states, e.out, e.dim, e.n_states,
-                                                        e.accumulate, stream);
+        fp_status const r = fprt::launch_op_apply_tiled(sp.tt, sp.at, sp.geo, e.dtype, e.states, e.out, e.dim,
+                                                        e.n_states, e.accumulate, stream);
         if (r != FP_OK)
             return r;
     }
@@ -382,6 +383,7 @@ fp_status build(fp_hip_batch *b, hipStream_t stream, bool columns)
         op.accumulate = e.accumulate ? 1u : 0u;
         fprt::TileGeom geo{};
         fprt::TileTables *tt = nullptr;
+        fprt::TileAddr at;
         bool const column_shape = column_candidate(e);
         auto to_columns = [&] {
             column_entries.push_back(fprt::ColumnEntry{
@@ -407,7 +409,7 @@ fp_status build(fp_hip_batch *b, hipStream_t stream, bool columns)
             if (ts == FP_OK && tt)
                 ts = fprt::check_tile_fit(tt, geo, e.dtype, fpa::kTileBytes);
             if (ts == FP_OK && tt)
-                ts = fprt::tile_device(o, tt, stream);
+                ts = fprt::tile_device(o, tt, stream, &at);
             if (ts == FP_OK && tt)
                 ts = fprt::apply_tiled_attributes();
             if (ts != FP_OK)
@@ -415,7 +417,7 @@ fp_status build(fp_hip_batch *b, hipStream_t stream, bool columns)
             if (tt)
             {
                 // launches of their own: no items in the persistent kernel
-                b->split.push_back(fp_hip_batch::Split{uint32_t(i), tt, geo});
+                b->split.push_back(fp_hip_batch::Split{uint32_t(i), tt, at, geo});
                 b->tiled_groups += tt->n_groups;
                 b->plan_bytes += double(entry_in_bytes(e)) * (3.0 * tt->n_groups - (e.accumulate ? 0.0 : 1.0));
                 op.sshift = 64u;
@@ -431,14 +433,14 @@ fp_status build(fp_hip_batch *b, hipStream_t stream, bool columns)
         uint32_t tiles = 0;
         if (tt)
         {
-            fp_status const us = fprt::tile_device(o, tt, stream);
+            fp_status const us = fprt::tile_device(o, tt, stream, &at);
             if (us != FP_OK)
                 return us;
             op.coset = 1;
             op.nc = coset_paired(e, geo) ? 2u : 1u;
-            op.groups = tt->groups;
-            op.btab = tt->btab;
-            op.astrs = static_cast<fpa::ApplyStr const *>(tt->strs);
+            op.groups = at.groups;
+            op.btab = at.btab;
+            op.astrs = static_cast<fpa::ApplyStr const *>(at.strs);
             op.lsb = geo.lsb;
             op.k = geo.k;
             op.d = geo.d;

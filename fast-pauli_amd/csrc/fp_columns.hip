@@ -99,8 +99,6 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
 {
     *done = false;
     bool const c64 = dtype != FP_C128;
-    if (!ws && stream_capturing(st)) // the slab may have to be allocated
-        return FP_OK;
     // one aligned state is a column already
     bool const in_place = n_states == 1 && (reinterpret_cast<uintptr_t>(states) & 15u) == 0;
     ColGeom const g = col_geom(ops, dtype, n_states, ws ? ws->bytes / 2 : kSlabBytes);
@@ -141,7 +139,8 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
             return FP_OK;
         std::lock_guard<std::mutex> lock(ops->tiles_mu);
         FP_HIP(hipMemcpyAsync(ws->base, tt->h.data(), tt->h.size(), hipMemcpyHostToDevice, st));
-        FP_HIP(hipEventRecord(tt->uploaded, st)); // the host image may be rebuilt only once this copy has read it
+        if (!stream_capturing(st)) // the host image may be rebuilt only once this copy has read it
+            FP_HIP(hipEventRecord(tt->uploaded, st));
         d_tables = static_cast<unsigned char *>(ws->base);
         base = static_cast<unsigned char *>(ws->base) + table_bytes;
     }
@@ -154,9 +153,10 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
             (void)hipGetLastError();
             return FP_OK; // no room for the slab: the kernels that read the batch as it is
         }
-        if (s != FP_OK || (s = tile_device(ops, tt, st)) != FP_OK)
+        TileAddr at;
+        if (s != FP_OK || (s = tile_device(ops, tt, st, &at)) != FP_OK)
             return s;
-        d_tables = static_cast<unsigned char const *>(tt->d_mem);
+        d_tables = at.base;
         base = static_cast<unsigned char *>(scratch);
     }
     auto *partial = reinterpret_cast<fpk::Dbl2 *>(base + slab_bytes);

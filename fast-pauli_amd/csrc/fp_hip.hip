@@ -151,6 +151,7 @@ fp_status scratch_get(hipStream_t stream, size_t bytes, void **out)
     bool const capture = stream_capturing(stream);
     if (s.bytes < bytes)
     {
+        RelaxedCapture const relaxed(capture);
         size_t want = std::max<size_t>(bytes, size_t(1) << 20);
         if (s.ptr && (s.captured || capture))
         {

@@ -27,6 +27,29 @@ namespace fprt
 // Whether work on `stream` is being captured into a graph.
 bool stream_capturing(hipStream_t stream);
 
+// While `active`, the calling thread may allocate and wait for other streams although a stream
+// is being captured (in global or thread-local mode, which forbid both).
+class RelaxedCapture
+{
+  public:
+    explicit RelaxedCapture(bool active) : active_(active)
+    {
+        if (active_)
+            (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+    ~RelaxedCapture()
+    {
+        if (active_)
+            (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+    RelaxedCapture(RelaxedCapture const &) = delete;
+    RelaxedCapture &operator=(RelaxedCapture const &) = delete;
+
+  private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    bool active_;
+};
+
 // Per-stream device scratch of at least `bytes`; the pointer stays valid until
 // the next, larger request on the same stream, or, handed out while the stream is
 // captured, until the stream is destroyed.  Callers hold a StreamGuard for
@@ -136,17 +159,28 @@ struct TileTables
     void *d_mem = nullptr;
     size_t cap = 0;
     hipEvent_t uploaded = nullptr; // completes when the last upload has read `h`
-    fpt::TileGroup *groups = nullptr;
-    uint64_t *btab = nullptr;
-    void *chunks = nullptr;
-    void *strs = nullptr;
-    fpt::ShStr *sh = nullptr; // shared-leader string records (expectation tables)
+    // the copy that captured calls use: written before any graph that holds it can run, and not
+    // by calls on streams
+    void *d_captured = nullptr;
+    bool captured = false;
 };
+
+// Device addresses of a table image.
+struct TileAddr
+{
+    unsigned char const *base = nullptr;
+    fpt::TileGroup const *groups = nullptr;
+    uint64_t const *btab = nullptr;
+    void const *chunks = nullptr;
+    void const *strs = nullptr;
+    fpt::ShStr const *sh = nullptr; // shared-leader string records (expectation tables)
+};
+TileAddr tile_addr(TileTables const *t, void const *mem);
 
 // `wht_min`: for kTilesEvMatrix, the smallest class evaluated through a transform (part of the key)
 fp_status tile_tables(fp_hip_ops const *ops, int kind, uint32_t k, uint32_t dh, TileTables **out,
                       uint32_t wht_min = 0);
-fp_status tile_device(fp_hip_ops const *ops, TileTables *t, hipStream_t stream);
+fp_status tile_device(fp_hip_ops const *ops, TileTables *t, hipStream_t stream, TileAddr *at);
 // The tables were cut for `geo`, and one tile of `geo` fits `tile_bytes` of LDS.
 fp_status check_tile_fit(TileTables const *tt, TileGeom const &geo, int dtype, size_t tile_bytes);
 void invalidate_tiles(fp_hip_ops *ops);
@@ -175,8 +209,8 @@ fp_status run_op_apply_tiled(fp_hip_ops const *ops, int dtype, void const *state
                              void const *weights = nullptr);
 // The launches of run_op_apply_tiled (one per string group) on tables already on the
 // device; enqueues nothing else, so a graph capture may record it.
-fp_status launch_op_apply_tiled(TileTables const *tt, TileGeom const &geo, int dtype, void const *states, void *out,
-                                size_t dim, size_t n_states, int accumulate, hipStream_t st,
+fp_status launch_op_apply_tiled(TileTables const *tt, TileAddr const &at, TileGeom const &geo, int dtype,
+                                void const *states, void *out, size_t dim, size_t n_states, int accumulate, hipStream_t st,
                                 void const *weights = nullptr);
 // Sets the tiled apply kernels' LDS limit (once per process).
 fp_status apply_tiled_attributes();
@@ -192,7 +226,7 @@ fp_status run_op_expect(fp_hip_ops const *ops, int dtype, void const *states, vo
                         int accumulate, hipStream_t st, Workspace const *ws = nullptr);
 // PauliOp expectation on state columns (fp_columns.hpp).  *done = false, with nothing
 // enqueued, when it cannot run here (no room for the transposed slab in the workspace or on
-// the device, or the stream is being captured): the caller takes another kernel.
+// the device): the caller takes another kernel.
 bool ev_columns_eligible(fp_hip_ops const *ops, int dtype, size_t n_states);
 fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *states, void *out, size_t dim,
                                 size_t n_states, int accumulate, hipStream_t st, Workspace const *ws, bool *done);

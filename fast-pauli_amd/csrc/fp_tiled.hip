@@ -118,22 +118,68 @@ fp_status tile_tables(fp_hip_ops const *ops, int kind, uint32_t k, uint32_t dh, 
     t->o_sh = img.o_sh;
     t->h = std::move(img.h);
     t->on_device = false;
+    t->captured = false;
     t->valid = true;
     *out = t;
     return FP_OK;
 }
 
+TileAddr tile_addr(TileTables const *t, void const *mem)
+{
+    auto const *base = static_cast<unsigned char const *>(mem);
+    return TileAddr{base,
+                    reinterpret_cast<fpt::TileGroup const *>(base),
+                    reinterpret_cast<uint64_t const *>(base + t->o_btab),
+                    base + t->o_chunks,
+                    base + t->o_strs,
+                    reinterpret_cast<fpt::ShStr const *>(base + t->o_sh)};
+}
+
+namespace
+{
+
+// The device copy for a call that is being captured, complete on return.  A copy recorded into
+// the graph would not make the tables current for anybody else, and HIP ends a capture in which
+// an event of the captured stream is waited for: so neither the streams' copy nor its event will
+// do (an expectation warmed by an eager call on its stream could not be captured).
+fp_status tile_device_captured(TileTables *t, TileAddr *at)
+{
+    RelaxedCapture const relaxed(true);
+    if (!t->captured)
+    {
+        if (t->d_captured) // of graphs captured before the set was re-targeted
+            FP_HIP(hipFree(t->d_captured));
+        t->d_captured = nullptr;
+        FP_HIP(hipMalloc(&t->d_captured, t->h.size()));
+        hipStream_t own = nullptr;
+        FP_HIP(hipStreamCreateWithFlags(&own, hipStreamNonBlocking));
+        hipError_t e = hipMemcpyAsync(t->d_captured, t->h.data(), t->h.size(), hipMemcpyHostToDevice, own);
+        hipError_t const es = hipStreamSynchronize(own);
+        (void)hipStreamDestroy(own);
+        FP_HIP(e);
+        FP_HIP(es);
+        t->captured = true;
+    }
+    *at = tile_addr(t, t->d_captured);
+    return FP_OK;
+}
+
+} // namespace
+
 // Makes the device copy of `t` current for kernels on `stream`: reuses its
 // device memory when large enough, uploads asynchronously on `stream` and
 // records an event that guards the host image.
-fp_status tile_device(fp_hip_ops const *ops, TileTables *t, hipStream_t stream)
+fp_status tile_device(fp_hip_ops const *ops, TileTables *t, hipStream_t stream, TileAddr *at)
 {
     std::lock_guard<std::mutex> lock(ops->tiles_mu);
+    if (stream_capturing(stream))
+        return tile_device_captured(t, at);
     if (t->on_device)
     {
         // the upload may have been issued on another stream: order this one after it
         if (t->uploaded)
             FP_HIP(hipStreamWaitEvent(stream, t->uploaded, 0));
+        *at = tile_addr(t, t->d_mem);
         return FP_OK;
     }
     size_t const total = t->h.size();
@@ -152,13 +198,8 @@ fp_status tile_device(fp_hip_ops const *ops, TileTables *t, hipStream_t stream)
         FP_HIP(hipEventCreateWithFlags(&t->uploaded, hipEventDisableTiming));
     FP_HIP(hipMemcpyAsync(t->d_mem, t->h.data(), total, hipMemcpyHostToDevice, stream));
     FP_HIP(hipEventRecord(t->uploaded, stream));
-    auto *base = static_cast<unsigned char *>(t->d_mem);
-    t->groups = reinterpret_cast<fpt::TileGroup *>(base);
-    t->btab = reinterpret_cast<uint64_t *>(base + t->o_btab);
-    t->chunks = base + t->o_chunks;
-    t->strs = base + t->o_strs;
-    t->sh = reinterpret_cast<fpt::ShStr *>(base + t->o_sh);
     t->on_device = true;
+    *at = tile_addr(t, t->d_mem);
     return FP_OK;
 }
 
@@ -169,6 +210,7 @@ void invalidate_tiles(fp_hip_ops *ops)
     {
         t.valid = false;
         t.on_device = false;
+        t.captured = false;
     }
 }
 
@@ -184,6 +226,8 @@ void release_tiles(fp_hip_ops *ops)
         }
         if (t.d_mem)
             (void)hipFree(t.d_mem);
+        if (t.d_captured)
+            (void)hipFree(t.d_captured);
     }
     ops->tiles.clear();
 }
@@ -256,11 +300,7 @@ fp_status run_op_expect_tiled(fp_hip_ops const *ops, int dtype, void const *stat
         return s;
     if ((s = check_tile_fit(tt, geo, dtype, size_t(geo.tile_kb) << 10)) != FP_OK)
         return s;
-    // device addresses of the tables: their own device copy, or the workspace's head
-    fpt::TileGroup const *d_groups;
-    uint64_t const *d_btab;
-    void const *d_chunks, *d_strs;
-    fpt::ShStr const *d_sh;
+    TileAddr at; // the tables' own device copy, or the workspace's head
     size_t const table_bytes = (tt->h.size() + 255) / 256 * 256;
     if (ws)
     {
@@ -269,25 +309,14 @@ fp_status run_op_expect_tiled(fp_hip_ops const *ops, int dtype, void const *stat
                         table_bytes, ws->bytes);
         std::lock_guard<std::mutex> lock(ops->tiles_mu);
         FP_HIP(hipMemcpyAsync(ws->base, tt->h.data(), tt->h.size(), hipMemcpyHostToDevice, st));
-        // the host image may be rebuilt only once this copy has read it
-        FP_HIP(hipEventRecord(tt->uploaded, st));
-        auto *base = static_cast<unsigned char *>(ws->base);
-        d_groups = reinterpret_cast<fpt::TileGroup const *>(base);
-        d_btab = reinterpret_cast<uint64_t const *>(base + tt->o_btab);
-        d_chunks = base + tt->o_chunks;
-        d_strs = base + tt->o_strs;
-        d_sh = reinterpret_cast<fpt::ShStr const *>(base + tt->o_sh);
+        // the host image may be rebuilt only once this copy has read it (a captured copy runs with
+        // its graph, and no wait outside could name it)
+        if (!stream_capturing(st))
+            FP_HIP(hipEventRecord(tt->uploaded, st));
+        at = tile_addr(tt, ws->base);
     }
-    else
-    {
-        if ((s = tile_device(ops, tt, st)) != FP_OK)
-            return s;
-        d_groups = tt->groups;
-        d_btab = tt->btab;
-        d_chunks = tt->chunks;
-        d_strs = tt->strs;
-        d_sh = tt->sh;
-    }
+    else if ((s = tile_device(ops, tt, st, &at)) != FP_OK)
+        return s;
     uint64_t const n_cosets = uint64_t(dim) >> geo.d;
     uint32_t const chunks_y = uint32_t((n_states + (size_t(1) << geo.lsb) - 1) >> geo.lsb);
     if (chunks_y > 65535u)
@@ -385,9 +414,9 @@ fp_status run_op_expect_tiled(fp_hip_ops const *ops, int dtype, void const *stat
                 if (mode == 2 && pack)
                     kfn = &fpt::k_op_expect_tiled<T, false, 64, 3>;
             hipLaunchKernelGGL(kfn, grid, dim3(TKB * 8), lds, st, typed_states, uint64_t(n_states), sshift, geo.lsb,
-                               geo.k, geo.d, ranges, uint32_t(n_parts), chunks_y, n_cosets, d_groups, d_btab,
-                               static_cast<fpt::TileChunk const *>(d_chunks),
-                               static_cast<fpt::TileStr const *>(d_strs), d_sh, partial);
+                               geo.k, geo.d, ranges, uint32_t(n_parts), chunks_y, n_cosets, at.groups, at.btab,
+                               static_cast<fpt::TileChunk const *>(at.chunks),
+                               static_cast<fpt::TileStr const *>(at.strs), at.sh, partial);
             FP_LAUNCHED();
         }
         hipLaunchKernelGGL(fpk::k_reduce_partials<T>, dim3(uint32_t(n_states)), dim3(fpk::kBlock), 0, st, partial,
@@ -480,8 +509,9 @@ fp_status apply_tiled_attributes()
     return FP_OK;
 }
 
-fp_status launch_op_apply_tiled(TileTables const *tt, TileGeom const &geo, int dtype, void const *states, void *out,
-                                size_t dim, size_t n_states, int accumulate, hipStream_t st, void const *weights)
+fp_status launch_op_apply_tiled(TileTables const *tt, TileAddr const &at, TileGeom const &geo, int dtype,
+                                void const *states, void *out, size_t dim, size_t n_states, int accumulate, hipStream_t st,
+                                void const *weights)
 {
     uint64_t const n_cosets = uint64_t(dim) >> geo.d;
     uint32_t const chunks_y = uint32_t((n_states + (size_t(1) << geo.lsb) - 1) >> geo.lsb);
@@ -509,7 +539,7 @@ fp_status launch_op_apply_tiled(TileTables const *tt, TileGeom const &geo, int d
     if (as != FP_OK)
         return as;
     dim3 const grid(uint32_t(blocks_x), chunks_y);
-    auto const *strs = static_cast<fpa::ApplyStr const *>(tt->strs);
+    auto const *strs = static_cast<fpa::ApplyStr const *>(at.strs);
     bool const wtd = weights != nullptr;
     for (uint32_t g = 0; g < tt->n_groups; ++g)
     {
@@ -523,7 +553,7 @@ fp_status launch_op_apply_tiled(TileTables const *tt, TileGeom const &geo, int d
                                          : &fpa::k_op_apply_tiled<double, false, false, false>);
             hipLaunchKernelGGL(kfn, grid, dim3(fpa::kThreads), fpa::kTileBytes, st, static_cast<V const *>(states),
                                static_cast<V *>(out), uint64_t(n_states), sshift, geo.lsb, geo.k, geo.d, n_cosets,
-                               tt->groups + g, tt->btab, strs, init_zero, static_cast<double const *>(weights));
+                               at.groups + g, at.btab, strs, init_zero, static_cast<double const *>(weights));
         }
         else
         {
@@ -539,7 +569,7 @@ fp_status launch_op_apply_tiled(TileTables const *tt, TileGeom const &geo, int d
                                       : &fpa::k_op_apply_tiled<float, false, false, false>));
             hipLaunchKernelGGL(kfn, grid, dim3(fpa::kThreads), fpa::kTileBytes, st, static_cast<V const *>(states),
                                static_cast<V *>(out), uint64_t(n_states), sshift, geo.lsb, geo.k, geo.d, n_cosets,
-                               tt->groups + g, tt->btab, strs, init_zero, static_cast<float const *>(weights));
+                               at.groups + g, at.btab, strs, init_zero, static_cast<float const *>(weights));
         }
         FP_LAUNCHED();
     }
@@ -558,9 +588,10 @@ fp_status run_op_apply_tiled(fp_hip_ops const *ops, int dtype, void const *state
         return s;
     if ((s = check_tile_fit(tt, geo, dtype, fpa::kTileBytes)) != FP_OK)
         return s;
-    if ((s = tile_device(ops, tt, st)) != FP_OK)
+    TileAddr at;
+    if ((s = tile_device(ops, tt, st, &at)) != FP_OK)
         return s;
-    return launch_op_apply_tiled(tt, geo, dtype, states, out, dim, n_states, accumulate, st, weights);
+    return launch_op_apply_tiled(tt, at, geo, dtype, states, out, dim, n_states, accumulate, st, weights);
 }
 
 // ---------------------------------------------------------------------------
@@ -617,8 +648,8 @@ size_t ev_coset_scratch_bytes(fp_hip_ops const *ops, int dtype, size_t dim, size
 }
 
 template <class T>
-fp_status launch_ev_coset(fp_hip_ops const *ops, TileTables *tt, CosetGeom const &g, void const *states,
-                          void *ev, size_t dim, size_t n_states, void *scratch, hipStream_t st)
+fp_status launch_ev_coset(fp_hip_ops const *ops, TileTables const *tt, TileAddr const &at, CosetGeom const &g,
+                          void const *states, void *ev, size_t dim, size_t n_states, void *scratch, hipStream_t st)
 {
     typedef typename fpk::VecOf<T, 1>::type V;
     V *transposed = static_cast<V *>(scratch);
@@ -646,8 +677,8 @@ fp_status launch_ev_coset(fp_hip_ops const *ops, TileTables *tt, CosetGeom const
         return fail(FP_ERR_RUNTIME, "coset column and transform buffers (%zu bytes) exceed the LDS", lds);
     dim3 const grid(uint32_t(n_states), gy, tt->n_groups * g.n_cos);
     hipLaunchKernelGGL(fpl::k_ev_coset<T>, grid, dim3(fpl::kThreads), lds, st, transposed, uint64_t(dim), g.d, g.k,
-                       g.n_cos, tt->groups, tt->btab, static_cast<fpl::EvChunk const *>(tt->chunks),
-                       static_cast<fpl::EvStr const *>(tt->strs), uint64_t(n_states), uint64_t(ops->n_strings),
+                       g.n_cos, at.groups, at.btab, static_cast<fpl::EvChunk const *>(at.chunks),
+                       static_cast<fpl::EvStr const *>(at.strs), uint64_t(n_states), uint64_t(ops->n_strings),
                        partial);
     FP_LAUNCHED();
     uint64_t const total = uint64_t(ops->n_strings) * n_states;
@@ -666,13 +697,14 @@ fp_status run_ev_coset(fp_hip_ops const *ops, int dtype, void const *states, voi
                               wht_min_strings(dtype == FP_C128 ? kWhtMinCosetC128 : fpl::kWhtMin));
     if (s != FP_OK)
         return s;
-    if ((s = tile_device(ops, tt, st)) != FP_OK)
+    TileAddr at;
+    if ((s = tile_device(ops, tt, st, &at)) != FP_OK)
         return s;
     if (tt->n_groups * g.n_cos > 65535u)
         return fail(FP_ERR_INVALID_ARGUMENT, "too many string groups for the coset kernel");
     if (dtype == FP_C128)
-        return launch_ev_coset<double>(ops, tt, g, states, ev, dim, n_states, scratch, st);
-    return launch_ev_coset<float>(ops, tt, g, states, ev, dim, n_states, scratch, st);
+        return launch_ev_coset<double>(ops, tt, at, g, states, ev, dim, n_states, scratch, st);
+    return launch_ev_coset<float>(ops, tt, at, g, states, ev, dim, n_states, scratch, st);
 }
 
 } // namespace fprt

@@ -171,8 +171,10 @@ fp_status fp_hip_op_expectation(fp_hip_ops const *ops, int dtype, void const *st
  * state made one contiguous column (a transposed copy in the stream's scratch, at most 128 MiB
  * at a time; a single aligned state as it is), tiles of it held in registers and LDS.  No
  * counterpart in the reference.  Where the copy has no room (device memory, or the static
- * workspace), and in fp_hip_op_expectation on a stream that is being captured, the call runs
- * the kernel of fp_hip_op_expectation_plan instead. */
+ * workspace) the call runs the kernel of fp_hip_op_expectation_plan instead.  A captured
+ * fp_hip_op_expectation runs the kernels of the eager call; its graph holds the stream's scratch
+ * (until the stream is destroyed) and the set's tables, so its replays are ordered by the caller
+ * with other calls on that stream and end before the set is re-targeted. */
 fp_status fp_hip_op_expectation_columns(fp_hip_ops const *ops, int dtype, size_t dim, size_t n_states,
                                         int *columns);
 

@@ -280,3 +280,56 @@ def test_captured_scratch_outlives_larger_calls(hip, monkeypatch):
         assert np.array_equal(d_big.to_array(np.complex128, phi.shape), H.op_apply(big, phi, C128))
     graph.destroy()
     stream.destroy()
+
+
+@pytest.mark.parametrize("mode", [0, 2], ids=["global", "relaxed"])
+@pytest.mark.parametrize("warm", [True, False], ids=["warm", "cold"])
+@pytest.mark.parametrize("entry,dtype,n,N,S", [
+    ("fp_hip_op_expectation", C128, 14, 64, 40),   # columns
+    ("fp_hip_op_expectation", C64, 15, 70, 1),     # one state, read in place
+    ("fp_hip_op_expectation", C128, 14, 16, 16),   # coset-tiled
+    ("fp_hip_op_expectation", C128, 9, 1, 3),      # streaming
+    ("fp_hip_op_expectation_noalloc", C128, 14, 64, 40),
+    ("fp_hip_op_apply", C128, 10, 40, 16),         # one column made of the batch
+    ("fp_hip_op_apply", C64, 14, 100, 80),         # transposed columns: streaming in the graph
+    ("fp_hip_op_apply", C128, 14, 100, 300),       # transposed columns: coset-tiled in the graph
+    ("fp_hip_summed_apply_weighted", C128, 10, 50, 3),
+])
+def test_captured_calls(hip, entry, dtype, n, N, S, warm, mode):
+    """Captured on the stream that an eager call warmed, or without one: every replay, with eager
+    work on the set between them, gives the eager call's bits."""
+    H.say(f"captured {entry} n={n} N={N} S={S} dtype={dtype} warm={warm} mode={mode}")
+    K, cdt = 4, H.CDT[dtype]
+    codes = syn.random_codes(N, n, seed=n + N)
+    rng = np.random.default_rng(N)
+    weighted = entry == "fp_hip_summed_apply_weighted"
+    make = (lambda: _abi.Ops(codes, matrix=mat)) if weighted else (lambda: _abi.Ops(codes, coeffs))
+    mat, coeffs = rng.standard_normal((N, K)) + 0j, syn.random_coeffs(N, seed=N)
+    psi = syn.random_states(1 << n, S, seed=N).astype(cdt)
+    shape = (S,) if "expectation" in entry else psi.shape
+    d_in = _abi.DeviceBuffer.from_array(psi)
+    d_data = _abi.DeviceBuffer.from_array(rng.standard_normal((K, S)).astype(np.float64 if dtype == C128 else np.float32))
+    d_out = _abi.DeviceBuffer(int(np.prod(shape)) * np.dtype(cdt).itemsize)
+    args = [d_in.ptr] + ([d_data.ptr] if weighted else []) + [d_out.ptr, 1 << n, S, 0]
+
+    def run(ops, handle):
+        _abi.call(entry, ops.handle, dtype, *args, handle)
+
+    run(make(), None)  # another set, on another stream
+    _abi.synchronize()
+    want = d_out.to_array(cdt, shape)
+    ops, stream = make(), _abi.Stream()
+    if warm:
+        run(ops, stream.handle)
+        stream.synchronize()
+    graph = H.Graph(stream, lambda handle: run(ops, handle), mode)
+    for rep in range(3):
+        d_out.zero()
+        _abi.synchronize()
+        graph.replay()
+        assert np.array_equal(d_out.to_array(cdt, shape), want), rep
+        run(ops, stream.handle if rep else None)
+        _abi.synchronize()
+        assert np.array_equal(d_out.to_array(cdt, shape), want), rep
+    graph.destroy()
+    stream.destroy()
