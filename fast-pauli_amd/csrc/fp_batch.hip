@@ -85,13 +85,11 @@ struct fp_hip_batch
     unsigned char *d_columns = nullptr, *d_slab = nullptr;
     size_t cap_columns = 0, cap_slab = 0, slab_bytes = 0;
     bool use_columns = true; // batch_without_columns
-    hipStream_t last_stream = nullptr; // of the last launch that used the slabs,
-    bool last_ordered = false;         // whose last_done another stream can wait for
     double plan_bytes = 0.0; // state passes of the plan: coset groups, or one per string
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipStream_t capture_stream = nullptr;
-    hipEvent_t last_done = nullptr; // recorded after every launch
+    hipEvent_t last_done = nullptr; // recorded after every launch that is not being captured
     double est_cost = 0.0;
 };
 
@@ -866,20 +864,13 @@ fp_status fp_hip_batch_launch(fp_hip_batch *b, void *stream)
         if (r != FP_OK)
             return r;
     }
-    // Launches on two streams would share the slabs: the second waits for the first.  A launch
+    // Launches share the work counters and the slabs of columns: each waits for the one before
+    // it, whatever its stream (free on the same one; one handle may be several streams).  A launch
     // that is being captured neither waits nor is waited for: its graph's runs are the caller's
     // to order.
-    bool ordered = false;
-    if (!b->rounds.empty())
-    {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cap) == hipSuccess)
-            ordered = cap == hipStreamCaptureStatusNone;
-        else
-            (void)hipGetLastError();
-        if (ordered && b->last_ordered && b->last_stream != st)
-            FP_HIP(hipStreamWaitEvent(st, b->last_done, 0));
-    }
+    bool const capture = fprt::stream_capturing(st);
+    if (!capture && b->last_done)
+        FP_HIP(hipStreamWaitEvent(st, b->last_done, 0));
     if (b->use_graph)
         FP_HIP(hipGraphLaunch(b->exec, st));
     else
@@ -888,11 +879,11 @@ fp_status fp_hip_batch_launch(fp_hip_batch *b, void *stream)
         if (r != FP_OK)
             return r;
     }
+    if (capture)
+        return FP_OK;
     if (!b->last_done)
         FP_HIP(hipEventCreateWithFlags(&b->last_done, hipEventDisableTiming));
     FP_HIP(hipEventRecord(b->last_done, st));
-    b->last_ordered = ordered;
-    b->last_stream = st;
     return FP_OK;
 }
 

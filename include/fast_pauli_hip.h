@@ -375,6 +375,9 @@ fp_status fp_hip_batch_column_info(fp_hip_batch const *batch, size_t *n_entries,
  * last build gave up waiting for the previous string group (an internal error: its outputs
  * are then unspecified). */
 fp_status fp_hip_batch_check(fp_hip_batch *batch);
+/* A launch waits for the batch's previous one, also on another stream (they share counters and
+ * column buffers).  One that is being captured does not, nor is it waited for: the caller orders
+ * the runs of its graph with the batch's other launches. */
 fp_status fp_hip_batch_launch(fp_hip_batch *batch, void *stream);
 /* enabled = 1 (default): launches replay a captured hipGraph; 0: kernels are enqueued
  * directly (cheaper when every launch has new entries, as in a serving loop). */

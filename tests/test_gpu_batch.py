@@ -4,6 +4,8 @@ tolerance for expectation values), graph replays equal the eager result
 bit-exactly, and schedules change apply results not at all and expectation
 values only within rounding."""
 
+import threading
+
 import numpy as np
 import pytest
 
@@ -374,24 +376,122 @@ def test_column_entries_bit_exact(hip, graph):
     b.destroy()
 
 
-def test_column_launches_on_two_streams(hip):
-    """Launches of one batch on two streams share its column buffers: the later one waits."""
-    H.say("batch columns on two streams")
-    entries = [Entry(_abi.FP_BATCH_APPLY, 14, 64, 33, C64, False, seed=80),
-               Entry(_abi.FP_BATCH_APPLY, 15, 64, 40, C64, False, seed=81)]
-    refs = [e.alone() for e in entries]
+def _two_round_batch(graph):
+    """Two accumulating entries of different types: two rounds that use the same column buffers
+    for different states."""
+    entries = [Entry(_abi.FP_BATCH_APPLY, 14, 64, 33, C64, True, seed=80),
+               Entry(_abi.FP_BATCH_APPLY, 15, 64, 20, C128, True, seed=81)]
     b = Batch()
+    if not graph:
+        _abi.call("fp_hip_batch_set_graph", b.handle, 0)
     for e in entries:
         b.add(e.kind, e.ops, e.d_in.ptr, e.d_out.ptr, 1 << e.n, e.S, e.dtype, e.accumulate)
-    streams = [_abi.Stream(), _abi.Stream()]
-    b.launch(streams[0])
-    for i in range(1, 8):
-        b.launch(streams[i % 2])
+    return b, entries
+
+
+def _accumulated(b, entries, launches):
+    """The outputs after so many launches one after the other."""
+    for e in entries:
+        e.reset()
+    for _ in range(launches):
+        b.launch()
+        _abi.synchronize()
+    assert b.info()["column_entries"] == 2 and b.info()["column_rounds"] == 2
+    want = [e.result() for e in entries]
+    for e in entries:
+        e.reset()
+    _abi.synchronize()
+    return want
+
+
+class _Stall:
+    """Work on a stream that outlasts the batch's launches by far."""
+
+    def __init__(self):
+        self.a, self.b = _abi.DeviceBuffer(1 << 30), _abi.DeviceBuffer(1 << 30)
+
+    def enqueue(self, handle):
+        for _ in range(60):  # 20 ms
+            _abi.call("fp_hip_copy", self.b.ptr, self.a.ptr, 1 << 30, handle)
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_column_launches_on_two_streams(hip, graph):
+    """Launches of one batch on two streams share its column buffers: each waits for the one
+    before it, although that one's stream is still busy when it is launched, or destroyed since."""
+    H.say(f"batch columns on two streams graph={graph}")
+    b, entries = _two_round_batch(graph)
+    want = _accumulated(b, entries, 7)
+    streams, stall = [_abi.Stream(), _abi.Stream()], _Stall()
+    for _ in range(3):
+        ended = _abi.Event()
+        stall.enqueue(streams[0].handle)
+        b.launch(streams[0])
+        ended.record(streams[0])
+        b.launch(streams[1])
+        streams[1].synchronize()
+        assert ended.query(), "the second launch did not wait for the first"
     for s in streams:
-        s.synchronize()
-    assert b.info()["column_entries"] == 2
-    for e, r in zip(entries, refs):
-        assert np.array_equal(e.result(), r)
+        s.destroy()
+    b.launch()
+    _abi.synchronize()
+    for e, w in zip(entries, want):
+        assert np.array_equal(e.result(), w)
+    b.destroy()
+
+
+def test_column_launches_around_a_captured_one(hip):
+    """A captured launch between two eager ones leaves their order alone; its graph accumulates
+    like a launch."""
+    H.say("batch columns around a captured launch")
+    b, entries = _two_round_batch(False)
+    want = _accumulated(b, entries, 5)
+    streams, stall, ended = [_abi.Stream() for _ in range(3)], _Stall(), _abi.Event()
+    stall.enqueue(streams[0].handle)
+    b.launch(streams[0])
+    ended.record(streams[0])
+    graph = H.Graph(streams[1], lambda handle: b.launch(handle), mode=2)
+    b.launch(streams[2])
+    streams[2].synchronize()
+    assert ended.query(), "the launch after the captured one did not wait for the first"
+    for _ in range(3):
+        graph.replay()
+        _abi.synchronize()
+    for e, w in zip(entries, want):
+        assert np.array_equal(e.result(), w)
+    graph.destroy()
     b.destroy()
     for s in streams:
         s.destroy()
+
+
+def test_column_launches_of_one_handle_in_two_threads(hip):
+    """hipStreamPerThread (2) is one handle for two streams: the second launch waits."""
+    H.say("batch columns on per-thread streams")
+    b, entries = _two_round_batch(True)
+    want = _accumulated(b, entries, 2)
+    stall, ended = _Stall(), _abi.Event()
+    launched, leave, failed = threading.Event(), threading.Event(), []
+
+    def body():
+        try:
+            stall.enqueue(2)
+            b.launch(2)
+            ended.record(2)
+        except Exception as e:  # reported by the main thread
+            failed.append(e)
+        launched.set()
+        leave.wait(timeout=60)
+
+    t = threading.Thread(target=body)
+    t.start()
+    assert launched.wait(timeout=60) and not failed, failed
+    b.launch(2)
+    _abi.call("fp_hip_stream_synchronize", 2)
+    done = ended.query()
+    leave.set()
+    t.join()
+    assert done, "the second launch did not wait for the first"
+    for e, w in zip(entries, want):
+        assert np.array_equal(e.result(), w)
+    b.destroy()
