@@ -23,7 +23,6 @@ namespace
 constexpr size_t kSlabBytes = size_t(128) << 20;
 // Tiles per column: at most 2^8 (a class pairs every tile with another one).
 constexpr uint32_t kMaxTileBits = 8;
-constexpr double kResidentItems = 470.0, kTargetItems = 2000.0;
 
 size_t round256(size_t v)
 {
@@ -104,30 +103,12 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
     ColGeom const g = col_geom(ops, dtype, n_states, ws ? ws->bytes / 2 : kSlabBytes);
     if (ws && !in_place && g.slab * g.col_bytes > ws->bytes / 2)
         return FP_OK;
-    uint32_t const n_groups_max = (g.slab + g.per_group - 1) / g.per_group;
-    // String evaluations per item.  Little work: from 4, so many that the blocks all fit on the
-    // chip at once (two a CU, less a margin).  More: at least about 20, which pay the item's tile
-    // loads, and kTargetItems blocks (one state, whose columns the XCDs share: half).  Steps of a
-    // quarter keep the tables cached per set few.  us at 16 evaluations and more / now: n = 16, one
-    // complex128 state, N = 64 15.8 / 9.4, N = 1024 (513 blocks of 16) 19.7 / 15.6; n = 15 N = 200
-    // 12.6 / 8.1; n = 10 S = 50 N = 64 13.8 / 11.0.  Blocks wanted of the large ones: n = 18 S = 13
-    // N = 300 512 312 / 1000 246 / 1500 224 / 2000 214 / 3000 216; n = 18 S = 1 N = 1000 57 / 45 /
-    // 48 / 52 / 56; n = 14 S = 1000 is flat.
-    uint32_t const w = fpc::tile_bits(c64), n = uint32_t(ops->n_qubits);
-    double const work = double(ops->n_strings) * double(n_groups_max) *
-                        (n > w ? 0.5 * double(uint32_t(1) << (n - w)) : 0.6);
-    uint32_t per = 4;
-    while (per < 20 && work > (n > w ? kResidentItems : 0.85 * kResidentItems) * per) // (whole items per group)
-        per += per / 4;
-    while (per < 256 && work > (n_states == 1 ? 0.5 : 1.0) * kTargetItems * per)
-        per += per / 4;
+    uint32_t const per = column_item_size(c64, uint32_t(ops->n_qubits), ops->n_strings, n_states, g.slab);
     TileTables *tt = nullptr;
     fp_status s = tile_tables(ops, kTilesEvColumns, per, c64 ? 1u : 0u, &tt);
     if (s != FP_OK)
         return s;
     uint32_t const n_items = tt->n_groups;
-    if (uint64_t(n_items) * n_groups_max > 0x7fffffffu)
-        return FP_OK;
     size_t const slab_bytes = in_place ? 0 : round256(size_t(g.slab) * g.col_bytes);
     size_t const part_bytes = round256(size_t(n_items) * g.slab * sizeof(fpk::Dbl2));
     unsigned char *base = nullptr;

@@ -602,6 +602,32 @@ double record_cost(fpc::ColStr const &r)
 
 } // namespace
 
+// Little work: from 4 evaluations, so many that the blocks all fit on the
+// chip at once (two a CU, less a margin).  More: at least about 20, which pay the item's tile
+// loads, and kTargetItems blocks (one state, whose columns the XCDs share: half).  Steps of a
+// quarter keep the tables cached per set few.  us at 16 evaluations and more / now: n = 16, one
+// complex128 state, N = 64 15.8 / 9.4, N = 1024 (513 blocks of 16) 19.7 / 15.6; n = 15 N = 200
+// 12.6 / 8.1; n = 10 S = 50 N = 64 13.8 / 11.0.  Blocks wanted of the large ones: n = 18 S = 13
+// N = 300 512 312 / 1000 246 / 1500 224 / 2000 214 / 3000 216; n = 18 S = 1 N = 1000 57 / 45 /
+// 48 / 52 / 56; n = 14 S = 1000 is flat.  Items end at 256 evaluations, up to kMaxColumnItems.
+uint32_t column_item_size(bool c64, uint32_t n, size_t n_strings, size_t n_states, size_t slab)
+{
+    constexpr double kResidentItems = 470.0, kTargetItems = 2000.0;
+    uint32_t const w = fpc::tile_bits(c64);
+    size_t const per_group = n < w ? size_t(1) << (w - n) : 1;
+    double const groups = double((slab + per_group - 1) / per_group), tiles = n > w ? double(1u << (n - w)) : 1.0;
+    double const work = double(n_strings) * groups * (n > w ? 0.5 * tiles : 0.6);
+    uint32_t per = 4;
+    while (per < 20 && work > (n > w ? kResidentItems : 0.85 * kResidentItems) * per) // (whole items per group)
+        per += per / 4;
+    while (per < 256 && work > (n_states == 1 ? 0.5 : 1.0) * kTargetItems * per)
+        per += per / 4;
+    // (a tile's items: at most its evaluations, one a string, over `per`, and one)
+    while (per < 0x40000000u && tiles * (double(n_strings) / per + 1.0) * double(slab) > double(kMaxColumnItems))
+        per += per / 4;
+    return per;
+}
+
 fp_status build_column_image(StringTable const &st, bool c64, uint32_t per_item, TileImage &out)
 {
     uint32_t const w = fpc::tile_bits(c64);

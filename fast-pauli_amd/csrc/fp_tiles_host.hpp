@@ -83,6 +83,12 @@ fp_status build_tile_image(StringTable const &st, int kind, uint32_t k, uint32_t
 // string evaluations of a whole tile (n_groups items).
 fp_status build_column_image(StringTable const &st, bool c64, uint32_t per_item, TileImage &out);
 
+// The `per_item` for a launch on `slab` columns of 2^n rows (one state: n_states = 1).
+uint32_t column_item_size(bool c64, uint32_t n, size_t n_strings, size_t n_states, size_t slab);
+// (item, column) pairs of a launch: their partials are 64 MiB at most, and their blocks, of 512
+// threads, stay below the 2^32 threads of a launch, beyond which HIP runs a part of them only.
+constexpr uint64_t kMaxColumnItems = uint64_t(1) << 22;
+
 // An apply of a batch that runs on columns.  Addresses are device addresses: the states and
 // outputs, and the operator's masks (32 bits) and folded coefficients of its type.
 struct ColumnEntry

@@ -10,9 +10,11 @@
 // Both sums are FP64 over the same terms in another order: N 2^n terms of size
 // |c| |psi|^2, so 1e-12 relative to sum_s |c_s| <psi|psi> leaves a margin over
 // the 1e-16 sqrt(N 2^n) expected.
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstdio>
+#include <utility>
 #include <vector>
 
 #include "fp_tiles_host.hpp"
@@ -312,6 +314,46 @@ int round_cases(Rng &r)
     return n_cases;
 }
 
+// A launch on `slab` columns stays below 2^32 threads of 512-thread blocks, and its partials, one
+// an item and column, below 64 MiB: counted in the tables, and bounded for the largest sets.
+int item_cases(Rng &r)
+{
+    int n_cases = 0;
+    auto launch = [&](bool c64, size_t n, size_t N, size_t slab, uint64_t n_items) {
+        uint32_t const w = fpc::tile_bits(c64);
+        uint64_t const per_group = n < w ? uint64_t(1) << (w - n) : 1, groups = (slab + per_group - 1) / per_group;
+        ++n_cases;
+        if (n_items * groups * fpc::kThreads >= uint64_t(1) << 32 || n_items * slab > fprt::kMaxColumnItems)
+        {
+            ++g_failures;
+            std::fprintf(stderr, "FAIL launch c64=%d n=%zu strings=%zu slab=%zu: %llu items\n", int(c64), n, N, slab,
+                         static_cast<unsigned long long>(n_items));
+        }
+    };
+    for (auto const &[n, N] : {std::pair<size_t, size_t>{9, 2200000}, {12, 3000}, {15, 700}})
+    {
+        size_t const slab = (size_t(128) << 20) / (size_t(16) << n);
+        Set const s = make(n, N, 0, r);
+        fprt::TileImage im;
+        uint32_t const per = fprt::column_item_size(false, uint32_t(n), N, 100000, slab);
+        g_failures += fprt::build_column_image(s.table(), false, per, im) != FP_OK;
+        launch(false, n, N, slab, im.n_groups);
+        uint64_t const tiles = n > fpc::tile_bits(false) ? uint64_t(1) << (n - fpc::tile_bits(false)) : 1;
+        g_failures += im.n_groups > tiles * (N / per + 1);
+    }
+    for (bool c64 : {false, true})
+        for (size_t n = fpc::low_bits(c64); n <= fpc::tile_bits(c64) + 8; ++n)
+            for (size_t N = 8; N < (size_t(1) << 31); N = N * 3 + 1)
+                for (size_t states : {size_t(1), size_t(100), size_t(100000)})
+                {
+                    size_t const slab = std::min((size_t(128) << 20) / ((c64 ? size_t(8) : size_t(16)) << n), states);
+                    uint64_t const tiles = n > fpc::tile_bits(c64) ? uint64_t(1) << (n - fpc::tile_bits(c64)) : 1;
+                    uint32_t const per = fprt::column_item_size(c64, uint32_t(n), N, states, slab);
+                    launch(c64, n, N, slab, tiles * (N / per + 1));
+                }
+    return n_cases;
+}
+
 } // namespace
 
 int main()
@@ -340,6 +382,7 @@ int main()
                 }
         }
     n_cases += round_cases(r);
+    n_cases += item_cases(r);
     // sizes the kernel does not take
     Set const small = make(fpc::low_bits(false) - 1, 4, 0, r), large = make(fpc::tile_bits(false) + 13, 4, 0, r);
     fprt::TileImage im;

@@ -61,6 +61,20 @@ def test_expectation_on_columns_several_slabs(hip, monkeypatch):
     assert H.ev_scaled_err(got, _oracle(codes, coeffs, psi), coeffs, psi) <= 1e-12
 
 
+def test_expectation_of_millions_of_strings(hip):
+    """Strings and columns whose items at their usual size would make a launch of more than 2^32
+    threads, of which HIP runs a part: larger items instead."""
+    n, N, S = 9, 2_200_000, 16384
+    H.say(f"expectation on columns n={n} N={N} S={S}")
+    codes, coeffs = syn.random_codes(N, n, seed=1), syn.random_coeffs(N, seed=1)
+    ops = _abi.Ops(codes, coeffs)
+    assert _abi.op_expectation_columns(ops, C128, 1 << n, S)
+    psi = syn.random_states(1 << n, S, seed=1)
+    got = H.op_expectation(ops, psi, C128)[[0, S // 2, S - 1]]
+    sample = np.ascontiguousarray(psi[:, [0, S // 2, S - 1]])
+    assert H.ev_scaled_err(got, _oracle(codes, coeffs, sample), coeffs, sample) <= 1e-12
+
+
 def test_expectation_on_columns_unaligned_state(hip, monkeypatch):
     """One complex64 state at 8 bytes past a 16-byte boundary (the ABI asks for 8): copied."""
     H.say("expectation on columns, unaligned state")
