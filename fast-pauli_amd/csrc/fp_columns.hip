@@ -29,25 +29,30 @@ size_t round256(size_t v)
     return (v + 255) / 256 * 256;
 }
 
-// Columns per tile of the expectation kernel and columns per slab.
+// Of an expectation: columns per tile and bytes per column.
 struct ColGeom
 {
-    uint32_t per_group, slab;
+    uint32_t per_group;
     size_t col_bytes;
 };
 
-ColGeom col_geom(fp_hip_ops const *ops, int dtype, size_t n_states, size_t slab_bytes)
+ColGeom col_geom(fp_hip_ops const *ops, int dtype)
 {
     bool const c64 = dtype != FP_C128;
     uint32_t const w = fpc::tile_bits(c64), n = uint32_t(ops->n_qubits);
-    ColGeom g{};
-    g.per_group = n < w ? 1u << (w - n) : 1u;
-    g.col_bytes = (size_t(1) << n) * (c64 ? 8u : 16u);
-    size_t cols = std::max<size_t>(1, std::min<size_t>(slab_bytes / g.col_bytes, n_states));
-    if (cols < n_states) // whole tiles, and as many columns on every XCD
-        cols = std::max<size_t>(cols / (8 * g.per_group) * (8 * g.per_group), std::min<size_t>(cols, g.per_group));
-    g.slab = uint32_t(std::min<size_t>(cols, 0x7fffffffu));
-    return g;
+    return ColGeom{n < w ? 1u << (w - n) : 1u, (size_t(1) << n) * (c64 ? 8u : 16u)};
+}
+
+// Columns of a slab that has room for `room`: whole tiles, and as many columns on every XCD.
+uint32_t slab_columns(ColGeom const &g, size_t n_states, size_t room)
+{
+    size_t cols = std::min(room, n_states);
+    if (cols < n_states)
+    {
+        size_t const whole = cols >= 8 * g.per_group ? 8 * g.per_group : g.per_group;
+        cols = std::max<size_t>(cols / whole * whole, std::min<size_t>(cols, g.per_group));
+    }
+    return uint32_t(std::min<size_t>(cols, 0x7fffffffu));
 }
 
 template <class T, int NS, bool IN>
@@ -100,24 +105,29 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
     bool const c64 = dtype != FP_C128;
     // one aligned state is a column already
     bool const in_place = n_states == 1 && (reinterpret_cast<uintptr_t>(states) & 15u) == 0;
-    ColGeom const g = col_geom(ops, dtype, n_states, ws ? ws->bytes / 2 : kSlabBytes);
-    if (ws && !in_place && g.slab * g.col_bytes > ws->bytes / 2)
-        return FP_OK;
-    uint32_t const per = column_item_size(c64, uint32_t(ops->n_qubits), ops->n_strings, n_states, g.slab);
+    ColGeom const g = col_geom(ops, dtype);
+    uint32_t slab = slab_columns(g, n_states, std::max<size_t>(1, kSlabBytes / g.col_bytes));
+    // (a workspace takes the same items on smaller slabs: the same sums)
+    uint32_t const per = column_item_size(c64, uint32_t(ops->n_qubits), ops->n_strings, n_states, slab);
     TileTables *tt = nullptr;
     fp_status s = tile_tables(ops, kTilesEvColumns, per, c64 ? 1u : 0u, &tt);
     if (s != FP_OK)
         return s;
     uint32_t const n_items = tt->n_groups;
-    size_t const slab_bytes = in_place ? 0 : round256(size_t(g.slab) * g.col_bytes);
-    size_t const part_bytes = round256(size_t(n_items) * g.slab * sizeof(fpk::Dbl2));
+    size_t const table_bytes = round256(tt->h.size());
+    if (ws)
+    {
+        size_t const per_column = (in_place ? 0 : g.col_bytes) + size_t(n_items) * sizeof(fpk::Dbl2);
+        if (ws->bytes < table_bytes + 256 + per_column)
+            return FP_OK;
+        slab = std::min(slab, slab_columns(g, n_states, (ws->bytes - table_bytes - 256) / per_column));
+    }
+    size_t const slab_bytes = in_place ? 0 : round256(slab * g.col_bytes);
+    size_t const part_bytes = round256(size_t(n_items) * slab * sizeof(fpk::Dbl2));
     unsigned char *base = nullptr;
     unsigned char const *d_tables = nullptr;
     if (ws)
     {
-        size_t const table_bytes = round256(tt->h.size());
-        if (table_bytes + slab_bytes + part_bytes > ws->bytes)
-            return FP_OK;
         std::lock_guard<std::mutex> lock(ops->tiles_mu);
         FP_HIP(hipMemcpyAsync(ws->base, tt->h.data(), tt->h.size(), hipMemcpyHostToDevice, st));
         if (!stream_capturing(st)) // the host image may be rebuilt only once this copy has read it
@@ -156,9 +166,9 @@ fp_status run_op_expect_columns(fp_hip_ops const *ops, int dtype, void const *st
         typedef decltype(T_tag) T;
         typedef typename fpk::VecOf<T, 1>::type V;
         typedef typename fpc::Piece<T>::type P;
-        for (size_t c0 = 0; c0 < n_states; c0 += g.slab)
+        for (size_t c0 = 0; c0 < n_states; c0 += slab)
         {
-            uint32_t const nc = uint32_t(std::min<size_t>(g.slab, n_states - c0));
+            uint32_t const nc = uint32_t(std::min<size_t>(slab, n_states - c0));
             P const *cols = static_cast<P const *>(states);
             if (!in_place)
             {

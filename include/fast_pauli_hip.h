@@ -184,8 +184,8 @@ fp_status fp_hip_op_expectation_columns(fp_hip_ops const *ops, int dtype, size_t
 /* fp_hip_op_expectation without any device allocation.  No counterpart in the reference: it is
  * for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  Same kernels, same results as fp_hip_op_expectation (identical bits
- * whenever the partials, and on state columns the transposed states, fit beside the tables
- * without fewer blocks or another kernel; otherwise a regrouped FP64 sum); the reduction
+ * whenever the partials fit beside the tables without fewer blocks, and on state columns whenever
+ * one column and its partials do; otherwise a regrouped FP64 sum); the reduction
  * partials, the transposed states and the string-group tables live in one static
  * FP_NOALLOC_SCRATCH_BYTES device array per GPU instead of library-allocated memory.  Shapes
  * whose tables and partials (tiled: groups x n_states x 16 B at least; streaming:

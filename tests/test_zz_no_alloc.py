@@ -62,6 +62,26 @@ def test_noalloc_matches_op_expectation(hip, dtype, kernel, n, N, S_big, S_small
         assert np.array_equal(got, ref)
 
 
+@pytest.mark.parametrize("dtype,n,N,S", [
+    (C128, 14, 1024, 700),  # 512 columns a slab, in the workspace fewer
+    (C128, 9, 300, 20000),  # 8 columns a tile, 16384 a slab
+    (C128, 20, 1000, 3),    # columns of 16 MiB: one at a time
+    (C64, 18, 300, 13),     # ragged, several columns a slab
+    (C64, 13, 90, 1),       # read in place
+])
+def test_noalloc_on_columns(hip, dtype, n, N, S):
+    """State columns, in slabs as small as the workspace makes them: the same items, the same sums."""
+    H.say(f"noalloc on columns n={n} N={N} S={S} dtype={dtype}")
+    dim = 1 << n
+    ops = _abi.Ops(syn.random_codes(N, n, seed=n + N), syn.random_coeffs(N, seed=n + N))
+    assert _abi.op_expectation_columns(ops, dtype, dim, S)
+    d_in = _abi.DeviceBuffer(dim * S * (16 if dtype == C128 else 8))
+    _abi.call("fp_hip_fill_states", dtype, d_in.ptr, dim, S, syn.gpu_seed(S), 1, None)
+    for acc0 in (None, syn.random_coeffs(S, seed=S)):
+        ref, got = _both(ops, d_in, dim, S, dtype, acc0=acc0)
+        assert np.array_equal(got, ref)
+
+
 def test_noalloc_rejects_oversized_partials(hip):
     """n_states x 16 B of partials per block above the static workspace: a clear
     error before any kernel runs."""
