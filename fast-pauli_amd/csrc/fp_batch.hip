@@ -39,6 +39,9 @@ struct BatchEntry
     uint64_t generation; // ops->generation the device tables were built from
 };
 
+// Default thresholds of the schedule.
+constexpr uint32_t kCosetMinKib = 256u << 10, kTiledMinKib = 64u << 10;
+
 struct fp_hip_batch
 {
     std::vector<BatchEntry> entries;
@@ -48,7 +51,7 @@ struct fp_hip_batch
     // those entries first: in a 256-entry batch of complex64 applies, the 15 entries of
     // 64 MiB and more took 33.4 ms as launches of their own, 38.9 ms as streaming items
     // and 43.9 ms as coset items.
-    fp_hip_batch_schedule sched{2048, 1u << 18, 4, FP_BATCH_ORDER_LARGEST_FIRST, 8, 256u << 10, 64u << 10};
+    fp_hip_batch_schedule sched{2048, 1u << 18, 4, FP_BATCH_ORDER_LARGEST_FIRST, 8, kCosetMinKib, kTiledMinKib};
     bool use_graph = true;
     // device tables, sized by capacity and reused across rebuilds
     bool built = false;
@@ -270,9 +273,10 @@ fp_status coset_plan(BatchEntry const &e, uint32_t min_kib, fprt::TileGeom *geo,
 constexpr size_t kRoundBytes = size_t(128) << 20;
 
 // Entries of at least this many bytes of states and terms (strings x elements) run on columns
-// whatever the schedule's thresholds; smaller ones where those leave them to the streaming items
-// and all the candidates of the batch are worth the launches of their rounds, three for each
-// variant (streaming items: about 1 ms for 1e9 terms).
+// where the schedule's thresholds would leave them to the streaming items, and while a caller has
+// not set those thresholds, before them (the 256 entries below: 18.5 ms, as coset-tiled launches
+// from 64 MiB 57.3).  Smaller ones where all the candidates of the batch are worth the launches of
+// their rounds, three for each variant (streaming items: about 1 ms for 1e9 terms).
 constexpr size_t kColumnsFirstBytes = size_t(4) << 20;
 constexpr double kColumnsFirstTerms = 3e7, kColumnsAllTerms = 5e8;
 
@@ -395,7 +399,8 @@ fp_status build(fp_hip_batch *b, hipStream_t stream, bool columns)
             op.n_tiles = 0;
             ops.push_back(op);
         };
-        if (column_shape && entry_in_bytes(e) >= kColumnsFirstBytes && entry_terms(e) >= kColumnsFirstTerms)
+        bool const column_size = entry_in_bytes(e) >= kColumnsFirstBytes && entry_terms(e) >= kColumnsFirstTerms;
+        if (column_shape && column_size && sc.tiled_min_kib == kTiledMinKib && sc.coset_min_kib == kCosetMinKib)
         {
             to_columns();
             continue;
@@ -463,7 +468,7 @@ fp_status build(fp_hip_batch *b, hipStream_t stream, bool columns)
             ops.push_back(op);
             continue;
         }
-        if (column_shape && column_terms >= kColumnsAllTerms)
+        if (column_shape && (column_size || column_terms >= kColumnsAllTerms))
         {
             to_columns();
             continue;

@@ -95,8 +95,10 @@ class Batch:
         _abi.call("fp_hip_batch_check", self.handle)
 
     def signature(self) -> str:
-        # the schedule layout is part of the key: cached choices of another layout are not reused
-        key = {"entries": sorted(self.entries), "schedule": [f for f, _ in _abi.BatchSchedule._fields_]}
+        # the schedule layout and what an untouched threshold stands for are part of the key: choices
+        # cached for another layout, or timed before entries ran on columns, are not reused
+        key = {"entries": sorted(self.entries), "schedule": [f for f, _ in _abi.BatchSchedule._fields_],
+               "default": "columns"}
         return hashlib.sha1(json.dumps(key).encode()).hexdigest()
 
     def autotune(self, stream=None, reps: int = 3, cache_path: str | None = None,

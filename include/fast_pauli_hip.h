@@ -367,9 +367,9 @@ fp_status fp_hip_batch_tiled_info(fp_hip_batch const *batch, size_t *n_entries, 
 /* Of the last build: apply entries run on columns (as fp_hip_op_apply does), and their rounds,
  * each of which copies at most 128 MiB of states into columns, applies, and copies the outputs
  * back, through buffers that the batch keeps (at most 256 MiB; without room for them those
- * entries run as the others do).  Entries of 4 MiB of states and more do so before the
- * thresholds of the schedule are looked at, smaller ones where those leave them to the
- * streaming items.  A server's batches do not. */
+ * entries run as the others do).  Entries of 4 MiB of states and more do so before the default
+ * thresholds of the schedule are looked at; with other thresholds, and smaller entries, only
+ * where those leave them to the streaming items.  A server's batches do not. */
 fp_status fp_hip_batch_column_info(fp_hip_batch const *batch, size_t *n_entries, size_t *n_rounds);
 /* Waits for the batch's last launch; FP_ERR_RUNTIME if a coset item of any launch since the
  * last build gave up waiting for the previous string group (an internal error: its outputs

@@ -376,6 +376,33 @@ def test_column_entries_bit_exact(hip, graph):
     b.destroy()
 
 
+def test_thresholds_that_a_caller_sets_hold(hip):
+    """Entries that run on columns by default run as coset-tiled launches or coset items where a
+    caller's thresholds say so, and on columns again where they leave them out."""
+    H.say("batch thresholds against columns")
+    entries = [Entry(_abi.FP_BATCH_APPLY, 14, 120, 33, C64, False, seed=70),
+               Entry(_abi.FP_BATCH_APPLY, 13, 200, 40, C128, True, seed=71)]
+    b = Batch()
+    for e in entries:
+        b.add(e.kind, e.ops, e.d_in.ptr, e.d_out.ptr, 1 << e.n, e.S, e.dtype, e.accumulate)
+    default = b.schedule
+    for sched, where in ((default, "column"), ({"tiled_min_kib": 1024}, "tiled"),
+                         ({"tiled_min_kib": 0, "coset_min_kib": 1024}, "coset"),
+                         ({"tiled_min_kib": 0, "coset_min_kib": 0}, "column"), (default, "column")):
+        b.schedule = {**default, **sched}
+        for e in entries:
+            e.reset()
+        b.launch()
+        _abi.synchronize()
+        info = b.info()
+        assert {k: info[k + "_entries"] for k in ("column", "tiled", "coset")} == \
+            {k: 2 * (k == where) for k in ("column", "tiled", "coset")}, (sched, info)
+        for e in entries:
+            assert np.array_equal(e.result(), e.alone())
+        b.check()
+    b.destroy()
+
+
 def _two_round_batch(graph):
     """Two accumulating entries of different types: two rounds that use the same column buffers
     for different states."""
