@@ -267,8 +267,12 @@ bool apply_lds_tiles(uint32_t n, uint64_t n_cols)
 //  1: a power-of-two state count (weighted: one state, whose weights are then one row) and a
 //     batch of at most 8 MiB (one state: 32 MiB), which the L2s and the Infinity Cache serve;
 //     beyond 4 MiB from 64 strings (n = 20, one complex128 state: N = 24 41.6 us streaming /
-//     45.9, N = 64 113 / 112).  us, streaming / column: n = 10, 128 states, 64 strings 14.1 / 6.9;
-//     n = 18, one state, 1000 strings 286 / 135.
+//     45.9, N = 64 113 / 112).  Below it from 2 strings, where both forms are one launch (n = 14,
+//     16 states: N = 2 3.6 / 3.6, N = 8 4.2 / 3.8, N = 16 6.4 / 5.2), but weighted from 8 (n = 14:
+//     N = 2..5 6.8 / 7.2, N = 8 7.6 / 7.3), and one complex64 state past 2 MiB, whose rows are 8
+//     bytes, from 16 (n = 19: N = 2 3.3 / 4.1, N = 12 5.6 / 6.5, N = 16 6.8 / 6.6, N = 24 10.9 /
+//     9.4; n = 18: N = 12 4.0 / 4.2, N = 24 6.3 / 5.5).  us, streaming / column: n = 10, 128 states,
+//     64 strings 14.1 / 6.9; n = 18, one state, 1000 strings 286 / 135.
 //  2: columns of at most 4 MiB (an XCD's L2), 8 MiB where the state count is not a power of two
 //     (the coset-tiled kernel is then at its slowest); enough work to pay the two transposed
 //     copies: from 32 strings and 3e7 (string, element) terms.  us, streaming or tiled / columns:
@@ -291,10 +295,14 @@ int apply_columns_route(fp_hip_ops const *ops, int dtype, size_t n_states, bool 
         return 0;
     size_t const elements = (size_t(1) << n) * n_states;
     bool const pow2 = (n_states & (n_states - 1)) == 0;
+    size_t const bytes = elements * esz;
     if (pow2 && (!weighted || n_states == 1) && elements >= 64 &&
-        elements * esz <= (n_states == 1 ? size_t(32) << 20 : size_t(8) << 20) &&
-        (elements * esz <= (size_t(4) << 20) || N >= 64 || forced))
-        return 1;
+        bytes <= (n_states == 1 ? size_t(32) << 20 : size_t(8) << 20))
+    {
+        size_t const narrow = dtype != FP_C128 && n_states == 1 && bytes > (size_t(2) << 20) ? 16 : 2;
+        if (forced || N >= (bytes > (size_t(4) << 20) ? 64 : std::max<size_t>(narrow, weighted ? 8 : 2)))
+            return 1;
+    }
     size_t const col_bytes = (size_t(1) << n) * esz;
     if (n < 6 || col_bytes > (size_t(8) << 20))
         return 0;

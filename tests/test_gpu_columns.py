@@ -210,6 +210,12 @@ def test_apply_columns_rule(hip, monkeypatch):
                           (20, 24, 1, False), (21, 96, 8, False), (10, 1, 128, False)):
         ops = _abi.Ops(syn.random_codes(N, n, seed=n))
         assert _abi.op_apply_columns(ops, C128, 1 << n, S) == want, (n, N, S)
+    # one complex64 state past 2 MiB, and weights of one state, pay from more strings on
+    for n, N, want in ((18, 2, True), (19, 15, False), (19, 16, True), (20, 63, False), (20, 64, True)):
+        ops = _abi.Ops(syn.random_codes(N, n, seed=n))
+        assert _abi.op_apply_columns(ops, C64, 1 << n, 1) == want, (n, N)
+    for N, want in ((7, False), (8, True)):
+        assert _abi.op_apply_columns(_abi.Ops(syn.random_codes(N, 10, seed=N)), C128, 1 << 10, 1, weighted=True) == want
     # weights per state: from 48 strings on small batches too
     for n, N, S, want in ((10, 48, 2, True), (10, 47, 2, False), (18, 48, 2, False), (18, 48, 3, True)):
         ops = _abi.Ops(syn.random_codes(N, n, seed=n))
