@@ -125,7 +125,9 @@ __device__ __forceinline__ void apply_columns(BlockOf bo, typename fpk::VecOf<T,
     uint32_t const g = n < kTile ? wave & ((1u << (n - kLow)) - 1u) : (p << (kTile - kLow)) | wave; // row >> kLow
     uint32_t const row0 = (g << kLow) | lane;
     V *oc = out + uint64_t(tc) * rows + row0;
-    uint32_t const a0 = ((wave << kLow) | lane) << kLv; // LDS address of slot 0
+    // LDS address of slot 0: the tile starts the workgroup's LDS, as the kernel has no static shared
+    // arrays (the launch checks it; adding the tile's address instead costs an instruction a read)
+    uint32_t const a0 = ((wave << kLow) | lane) << kLv;
     if constexpr (LDS)
     {
 #pragma unroll

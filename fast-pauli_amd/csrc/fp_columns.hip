@@ -224,12 +224,18 @@ fp_status launch_apply_columns(void const *cols, void *out, uint32_t n, uint32_t
         {
             static std::once_flag once;
             static hipError_t attr = hipSuccess;
+            static hipFuncAttributes fa{};
             std::call_once(once, [&] {
                 attr = hipFuncSetAttribute(reinterpret_cast<void const *>(kfn),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds));
+                if (attr == hipSuccess)
+                    attr = hipFuncGetAttributes(&fa, reinterpret_cast<void const *>(kfn));
             });
             if (attr != hipSuccess)
-                return fail(FP_ERR_RUNTIME, "hipFuncSetAttribute failed: %s", hipGetErrorString(attr));
+                return fail(FP_ERR_RUNTIME, "apply kernel attributes: %s", hipGetErrorString(attr));
+            if (fa.sharedSizeBytes != 0)
+                return fail(FP_ERR_RUNTIME, "the apply kernel's tile does not start its LDS: %zu static bytes",
+                            fa.sharedSizeBytes);
         }
         uint32_t const tiles = n > kTile ? 1u << (n - kTile) : 1u, per = n < kTile ? 1u << (kTile - n) : 1u;
         uint32_t const groups = (n_cols + per - 1) / per;
