@@ -340,9 +340,10 @@ def test_tiled_launch_entries_bit_exact(hip, graph):
 
 @pytest.mark.parametrize("graph", [True, False])
 def test_column_entries_bit_exact(hip, graph):
-    """Apply entries run on columns, in rounds of one slab after the other entries: IEEE-equal to the operator alone, both types, one and two states a row (an odd
-    last state), LDS tiles and direct columns, more than one round, accumulating, beside
-    streaming and expectation entries, over replays; re-targeted sets are picked up."""
+    """Apply entries run on columns, in rounds of one slab, after the other entries: IEEE-equal to
+    the operator alone, both types, one and two states a row (an odd last state), more than one
+    round, accumulating, beside streaming and expectation entries, over replays; re-targeted sets
+    are picked up."""
     H.say(f"batch columns graph={graph}")
     A, E = _abi.FP_BATCH_APPLY, _abi.FP_BATCH_EXPECT
     specs = [

@@ -224,6 +224,34 @@ def test_apply_columns_rule(hip, monkeypatch):
     assert not _abi.op_apply_columns(_abi.Ops(syn.random_codes(64, 10, seed=1)), C128, 1 << 10, 128)
 
 
+@pytest.mark.parametrize("dtype,n,S", [(C128, 12, 9), (C64, 15, 1), (C64, 13, 6)])
+def test_columns_follow_assign_and_coeffs(hip, monkeypatch, dtype, n, S):
+    """Re-targeted sets (more strings, fewer, others) and new coefficients: the expectation's cached
+    items and the apply's masks and coefficients are those of a fresh set."""
+    H.say(f"columns after assign / set_coeffs n={n} S={S} dtype={dtype}")
+    monkeypatch.setenv("FAST_PAULI_EV_KERNEL", "columns")
+    monkeypatch.setenv("FAST_PAULI_APPLY_KERNEL", "columns")
+    psi = syn.random_states(1 << n, S, seed=31).astype(H.CDT[dtype])
+    ops = _abi.Ops(syn.random_codes(64, n, seed=31), syn.random_coeffs(64, seed=31))
+
+    def same_as(fresh):
+        assert _abi.op_expectation_columns(ops, dtype, 1 << n, S) and _abi.op_apply_columns(ops, dtype, 1 << n, S)
+        assert np.array_equal(H.op_expectation(ops, psi, dtype), H.op_expectation(fresh, psi, dtype))
+        assert np.array_equal(H.op_apply(ops, psi, dtype), H.op_apply(fresh, psi, dtype))
+
+    same_as(_abi.Ops(syn.random_codes(64, n, seed=31), syn.random_coeffs(64, seed=31)))
+    for N, seed in ((300, 32), (40, 33), (300, 34)):
+        codes, coeffs = syn.random_codes(N, n, seed=seed), syn.random_coeffs(N, seed=seed)
+        ops.assign(codes, coeffs)
+        _abi.synchronize()
+        same_as(_abi.Ops(codes, coeffs))
+    coeffs = syn.random_coeffs(300, seed=35)
+    ops.set_coeffs(coeffs)
+    same_as(_abi.Ops(codes, coeffs))
+    want = _oracle(codes, coeffs, psi)
+    assert H.ev_scaled_err(H.op_expectation(ops, psi, dtype), want, coeffs, psi) <= (1e-12 if dtype == C128 else 1e-5)
+
+
 # ---------------------------------------------------------------------------
 # streams, threads and captured graphs
 # ---------------------------------------------------------------------------

@@ -37,17 +37,19 @@ def _both(ops, d_in, dim, S, dtype, acc0=None):
 
 @pytest.mark.parametrize("dtype", [C128, C64])
 @pytest.mark.parametrize("kernel,n,N,S_big,S_small", [
-    ("tiled", 20, 200, 16, 3),     # coset-tiled groups (the default for many strings)
+    ("tiled", 20, 200, 16, 3),     # coset-tiled groups
     ("tiled", 14, 64, 40, 7),      # ragged state counts
     ("stream", 12, 1, 9, 2),       # one string: the streaming kernel
 ])
-def test_noalloc_matches_op_expectation(hip, dtype, kernel, n, N, S_big, S_small):
+def test_noalloc_matches_op_expectation(hip, monkeypatch, dtype, kernel, n, N, S_big, S_small):
+    monkeypatch.setenv("FAST_PAULI_EV_KERNEL", kernel)  # not on columns
     dim = 1 << n
     tol = 1e-12 if dtype == C128 else 1e-5
     codes = syn.random_codes(N, n, seed=n + N)
     coeffs = syn.random_coeffs(N, seed=n + N)
     ops = _abi.Ops(codes, coeffs)
     for S in (S_big, S_small):  # the second call has the smaller input
+        assert not _abi.op_expectation_columns(ops, dtype, dim, S)
         plan = _abi.op_expectation_plan(ops, dtype, dim, S)
         H.say(f"noalloc vs op_expectation kernel={kernel} n={n} N={N} S={S} dtype={dtype} plan={plan}")
         assert plan["kernel"] == (_abi.FP_EV_TILED if kernel == "tiled" else _abi.FP_EV_STREAM)
