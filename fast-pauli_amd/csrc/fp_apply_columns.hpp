@@ -13,19 +13,21 @@
 // a per-lane offset (one XOR per string), a scalar offset per slot.  The sign is a per-lane bit,
 // a wave-uniform bit and one flip per slot, applied as the factor of the final multiply-add.
 //
-// Bound: 12 to 14 vector instructions per (string, 64 rows), 8 of them the unfused product and
-// sums, against 16 clocks of L1 for a gathered KiB (64 bytes a clock; 4 clocks from LDS) and the
-// scalar unit, which all four SIMDs share: whole rounds of strings run without a branch, on
+// Bound: 10 (LDS) to 12 vector instructions per (string, 64 rows), 8 of them the unfused product
+// and sums, against 16 clocks of L1 for a gathered KiB (64 bytes a clock; 4 clocks from LDS) and
+// the scalar unit, which all four SIMDs share: whole rounds of strings run without a branch, on
 // structure-of-arrays masks (wide scalar loads), and with one row a thread only a shift a string
 // is scalar.  Tests between the strings and masks split by scalar instructions made every wave
 // wait for its loads (n = 16, one complex128 state, 500 strings 40.6 us, now 19.3; n = 10, 128
-// states, 64 strings 8.5, now 6.9; n = 18, 13 complex64 states, 300 strings 524, now 397).  Two
+// states, 64 strings 10.9, now 8.1; n = 18, 13 complex64 states, 300 strings 524, now 397).  Two
 // shapes are built: one row a thread, partner rows gathered from L2 four or eight strings ahead;
-// and 2^13 rows a block in LDS (fp_columns.hip says which runs where).  Measured, row-major
-// kernels / columns, us: n = 10, 128 complex128 states, 64 strings 18.6 / 9.8; n = 18, one
-// complex128 state, 1000 strings 287 / 135; n = 20, 19 complex64 states, 512 strings 10990 / 5700
-// (8 MiB a column: past an XCD's L2); n = 14, 1000 complex128 states, 2000 strings, a weight per
-// string and state 29130 / 10800.
+// and 2^13 rows a block in LDS (fp_columns.hip says which runs where).  By its counters: n = 18,
+// one complex128 state, L1 76 % and vector issue 57 % busy; n = 14 with weights, from LDS,
+// vector issue 81 %; n = 20 complex64, half of the gathers miss the L2, whose 4 MiB hold half of
+// a column.  Measured, row-major kernels / columns, us: n = 10, 128 complex128 states, 64
+// strings 18.6 / 8.1; n = 18, one complex128 state, 1000 strings 287 / 141; n = 20, 19 complex64
+// states, 512 strings 10990 / 5640; n = 14, 1000 complex128 states, 2000 strings, a weight per
+// string and state 29130 / 10930.
 #pragma once
 
 #include <hip/hip_runtime.h>

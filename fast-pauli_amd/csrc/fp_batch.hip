@@ -267,9 +267,9 @@ fp_status coset_plan(BatchEntry const &e, uint32_t min_kib, fprt::TileGeom *geo,
     return FP_OK;
 }
 
-// Columns of a round: as many bytes of outputs again.  Both are in the Infinity Cache (256 MB)
-// when the next kernel of the round reads them (256 entries, 3 GB: 32 MiB 19.9 ms, 64 MiB 19.1,
-// 128 MiB 18.9, 256 MiB 19.2, 512 MiB 19.4).
+// Columns of a round: as many bytes of outputs again, which together fill the Infinity Cache
+// (256 MB).  256 entries, 3 GB: 32 MiB 19.9 ms, 64 MiB 19.1, 128 MiB 18.9, 256 MiB 19.2, 512 MiB
+// 19.4.
 constexpr size_t kRoundBytes = size_t(128) << 20;
 
 // Entries of at least this many bytes of states and terms (strings x elements) run on columns

@@ -18,8 +18,12 @@ using fprt::fail;
 namespace
 {
 
-// Transposed states kept at a time: a slab this size is still in the Infinity Cache
-// (256 MB) when the column kernel reads it.
+// Transposed states kept at a time (an apply keeps as much of outputs again).  The slab of an
+// expectation is still in the Infinity Cache (256 MB) when its kernel reads it; an apply's two fill
+// that cache.  us with 32 / 64 / 128 / 256 MiB: expectation n = 14, 1000 complex128 states, 1024
+// strings 1744 / 1661 / 1594 / 1571, n = 20, 20 states, 1000 strings 5138 / 5087 / 4484 / 4369;
+// apply n = 14, 1000 states, 500 strings 3277 / 3222 / 3162 / 3177, n = 20, 19 complex64 states, 512
+// strings 5959 / 5842 / 5762 / 5680.
 constexpr size_t kSlabBytes = size_t(128) << 20;
 // Tiles per column: at most 2^8 (a class pairs every tile with another one).
 constexpr uint32_t kMaxTileBits = 8;
@@ -207,8 +211,8 @@ namespace
 // straight from the column; or 2^13-row tiles in LDS, eight rows a thread.
 template <class T, int NS, bool WTD>
 fp_status launch_apply_columns(void const *cols, void *out, uint32_t n, uint32_t n_cols, uint32_t n_states,
-                               uint32_t const *xs, uint32_t const *zs, T const *cf, uint64_t cf_stride, uint32_t n_strings, uint32_t shift,
-                               int accumulate, bool lds, hipStream_t st)
+                               uint32_t const *xs, uint32_t const *zs, T const *cf, uint64_t cf_stride,
+                               uint32_t n_strings, uint32_t shift, int accumulate, bool lds, hipStream_t st)
 {
     typedef typename fpk::VecOf<T, NS>::type V;
     auto go = [&](auto e_tag, auto u_tag, auto th_tag, auto lds_tag) -> fp_status {
@@ -278,12 +282,12 @@ bool apply_lds_tiles(uint32_t n, uint64_t n_cols)
 //     N = 2..5 6.8 / 7.2, N = 8 7.6 / 7.3), and one complex64 state past 2 MiB, whose rows are 8
 //     bytes, from 16 (n = 19: N = 2 3.3 / 4.1, N = 12 5.6 / 6.5, N = 16 6.8 / 6.6, N = 24 10.9 /
 //     9.4; n = 18: N = 12 4.0 / 4.2, N = 24 6.3 / 5.5).  us, streaming / column: n = 10, 128 states,
-//     64 strings 14.1 / 6.9; n = 18, one state, 1000 strings 286 / 135.
+//     64 strings 18.6 / 8.1; n = 18, one state, 1000 strings 287 / 141.
 //  2: columns of at most 4 MiB (an XCD's L2), 8 MiB where the state count is not a power of two
 //     (the coset-tiled kernel is then at its slowest); enough work to pay the two transposed
 //     copies: from 32 strings and 3e7 (string, element) terms.  us, streaming or tiled / columns:
-//     n = 14, 1000 complex128 states, 500 strings 8500 / 3270; n = 20, 19 complex64 states, 512
-//     strings 10900 / 5710; but n = 12, 100 complex64 states, 64 strings (2.6e7 terms) 16.2 / 21.3
+//     n = 14, 1000 complex128 states, 500 strings 8500 / 3160; n = 20, 19 complex64 states, 512
+//     strings 10990 / 5640; but n = 12, 100 complex64 states, 64 strings (2.6e7 terms) 16.2 / 21.3
 //     and n = 20, 16 complex64 states, 64 strings 619 / 733.
 //     Weighted, whose row-major form reads a weight per string and element: also from 48 strings
 //     on fewer than 2^19 elements.  n = 10, 2 states, 89 strings 43.8 / 17.2; n = 12, 100 states, 48
@@ -383,7 +387,8 @@ fp_status run_apply_columns(fp_hip_ops const *ops, int dtype, int kind, void con
                 if (two)
                     return launch_apply_columns<T, 2, false>(states, out, n + shift - 1, 1, 1, xs, zs, coef, 0, N,
                                                              shift - 1, accumulate, false, st);
-            return weighted ? launch_apply_columns<T, 1, true>(states, out, n, 1, 1, xs, zs, w, N, N, 0, accumulate, false, st)
+            return weighted ? launch_apply_columns<T, 1, true>(states, out, n, 1, 1, xs, zs, w, N, N, 0, accumulate,
+                                                               false, st)
                             : launch_apply_columns<T, 1, false>(states, out, n + shift, 1, 1, xs, zs, coef, 0, N, shift,
                                                                 accumulate, false, st);
         }
@@ -472,7 +477,8 @@ fp_status launch_column_round(ColumnRound const &r, unsigned char const *tables,
         hipLaunchKernelGGL((fpc::k_columns_batch<T, NS, true>), dim3(r.in_blocks), dim3(256), 0, st, in, out,
                            copies(r.o_in), copy_ends(r.o_in_ends), r.n_in);
         FP_LAUNCHED();
-        hipLaunchKernelGGL((fpc::k_apply_columns_batch<T, NS>), dim3(r.blocks), dim3(256), 0, st, in, out, jobs, ends, segs, r.n_segs);
+        hipLaunchKernelGGL((fpc::k_apply_columns_batch<T, NS>), dim3(r.blocks), dim3(256), 0, st, in, out, jobs, ends,
+                           segs, r.n_segs);
         FP_LAUNCHED();
         hipLaunchKernelGGL((fpc::k_columns_batch<T, NS, false>), dim3(r.out_blocks), dim3(256), 0, st, in, out,
                            copies(r.o_out), copy_ends(r.o_out_ends), r.n_out);

@@ -14,15 +14,16 @@
 // for the three slot bits (and the sub bit), applied in a tree of FMAs.  The string's
 // coefficient is known, so its sum stays in the thread: no cross-lane sum per string.
 //
-// Bound: LDS reads (one wave read of 16 bytes per lane takes 4 clocks of a CU) and vector
-// issue (about 33 instructions per string and 8 slots), each 70 % busy at n = 14 (counters:
-// 4.03 clocks per read, no bank conflicts); a second pair of strings in flight gains nothing
+// Bound: LDS reads (one wave read of 16 bytes per lane takes 4 clocks of a CU) and vector issue
+// (about 33 instructions per string and 8 slots); at n = 14 they are 62 % and 64 % busy, scalar
+// issue 56 %, without bank conflicts, and a second pair of strings in flight gains nothing
 // there.  With few strings per class the tile loads are the larger part (n = 18, 13 complex64
-// states: vector issue 57 %).  Tiles of 64 KiB in 512-thread blocks, two to a CU, so that
-// one block's loads overlap the other's strings; 8 slots of 16 bytes keep 96-101 VGPRs, four
-// waves per SIMD.  Measured against the coset-tiled kernel (us): n = 14, 1024 strings, 1000
-// complex128 states 6320 -> 1595; n = 16, 1024 strings, one state 67 -> 19; n = 18, 300
-// strings, 13 complex64 states 361 -> 130.
+// states: vector issue 54 %, LDS 30 %).  Shares are of issue counters over the kernel's cycles,
+// an instruction taking four of its SIMD or of its CU's LDS.  Tiles of 64 KiB in 512-thread
+// blocks, two to a CU, so that one block's loads overlap the other's strings; 8 slots of 16
+// bytes keep 95 (complex64 99) VGPRs, four waves per SIMD.  Measured against the coset-tiled
+// kernel (us): n = 14, 1024 strings, 1000 complex128 states 6200 -> 1610; n = 16, 1024 strings,
+// one state 70 -> 15.4; n = 18, 300 strings, 13 complex64 states 373 -> 114.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -116,7 +116,8 @@ struct ColumnRound
 };
 
 // Cuts the entries into rounds of at most `slab_bytes` of columns of one variant, longest
-// operators first, so that the blocks of a round last about as long.  `used`: the bytes of columns of the largest round.
+// operators first, so that the blocks of a round last about as long.  `used`: the bytes of columns
+// of the largest round.
 void build_column_rounds(std::vector<ColumnEntry> const &entries, size_t slab_bytes,
                          std::vector<ColumnRound> &rounds, std::vector<unsigned char> &image, size_t &used);
 

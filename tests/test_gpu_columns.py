@@ -356,7 +356,8 @@ def test_captured_calls(hip, entry, dtype, n, N, S, warm, mode):
     psi = syn.random_states(1 << n, S, seed=N).astype(cdt)
     shape = (S,) if "expectation" in entry else psi.shape
     d_in = _abi.DeviceBuffer.from_array(psi)
-    d_data = _abi.DeviceBuffer.from_array(rng.standard_normal((K, S)).astype(np.float64 if dtype == C128 else np.float32))
+    data = rng.standard_normal((K, S)).astype(np.float64 if dtype == C128 else np.float32)
+    d_data = _abi.DeviceBuffer.from_array(data)
     d_out = _abi.DeviceBuffer(int(np.prod(shape)) * np.dtype(cdt).itemsize)
     args = [d_in.ptr] + ([d_data.ptr] if weighted else []) + [d_out.ptr, 1 << n, S, 0]
 
